@@ -1129,12 +1129,12 @@ static int build_k_append(const starkv_k_append_desc* d, KAppendArgs& a) {
   a.pos0_dev = d->pos0_device; a.err = d->error_flag;
   a.fmt = k.format;
   a.data = (void*)k.data; a.stride_b = k.stride_b;
-  a.scale = (void*)k.scale; a.sc_sb = k.scale_stride_b; a.sc_sh = k.scale_stride_h;
+  a.scale = (void*)k.scale; a.sc_sb = k.scale_stride_b; a.sc_sh = k.scale_stride_h; a.sc_ss = 1;
   const bool two = k.format == STARKV_FMT_INT4_REF && k.split > 0;
   a.split = two ? k.split : 128;
   a.a_int8 = two ? k.split_format == STARKV_FMT_INT8_SYM : k.format == STARKV_FMT_INT8_SYM;
   a.data2 = (void*)k.data2; a.stride2_b = k.stride2_b;
-  a.scale2 = (void*)k.scale2; a.sc2_sb = k.scale2_stride_b; a.sc2_sh = k.scale2_stride_h;
+  a.scale2 = (void*)k.scale2; a.sc2_sb = k.scale2_stride_b; a.sc2_sh = k.scale2_stride_h; a.sc2_ss = 1;
   for (int h = 0; h < k.n_kv_heads; ++h) {
     a.rank[h] = k.rank[h];
     a.off[h] = k.head_offset[h]; a.pitch[h] = k.pos_stride[h];

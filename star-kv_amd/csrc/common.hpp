@@ -120,10 +120,10 @@ struct KAppendArgs {
   int* err;                                         // optional: set to 1 when a row is skipped
   int fmt;                                          // STARKV_FMT_DENSE or a quantised format
   void* data; int64_t stride_b;                     // dense: elements; quantised: bytes
-  void* scale; int64_t sc_sb, sc_sh;
+  void* scale; int64_t sc_sb, sc_sh, sc_ss;         // scale of position s at + s * sc_ss
   int split, a_int8;                                // ranks [0, split) in data (int8 if a_int8)
   void* data2; int64_t stride2_b;                   // ranks [split, r) as int4
-  void* scale2; int64_t sc2_sb, sc2_sh;
+  void* scale2; int64_t sc2_sb, sc2_sh, sc2_ss;
   int rank[K_MAX_KV];
   int64_t off[K_MAX_KV], pitch[K_MAX_KV];
   int64_t off2[K_MAX_KV], pitch2[K_MAX_KV];

@@ -178,8 +178,370 @@ __global__ __launch_bounds__(256) void step_append_kernel(const StepAppendArgs a
   rope_apply_row<T>(a.r, blk * 256 + threadIdx.x);
 }
 
+// ---------------------------------------------------------------------------
+// Many rows at once (a prompt).  The row-per-wave kernels above read 2 bytes
+// per lane and spend most lanes on the short K rows; these read and write
+// whole 8-rank chunks.
+//
+// Bytes bound this work, and past them the divisions: 8 + 4 latent bytes per
+// 4 stored ones leave ~16 VALU operations per element at the copy rate, which
+// two correctly rounded divisions would take alone.  The codes need only the
+// quotient's rounding to an integer, so a chunk multiplies by the correctly
+// rounded reciprocal of its scale and corrects the product by its exact
+// residual.  Symmetric blocks: x and s have at most 11 significant bits, so
+// the quotient is a tie n + 1/2 exactly or lies 2^-19 away from it
+// (relatively), and one correction, exact at ties, rounds as the division
+// does.  Group-64: x - z has 24 bits; two corrections give the correctly
+// rounded quotient itself (Markstein's theorem: a faithful quotient and a
+// correctly rounded reciprocal).  A scale outside fp16's range divides.
+// Measured at B8 T2048 (32 heads, ranks sum 1640, Rv 1640, int8 K / group-64
+// V, 151 MB): 348 -> 55 us a call, 51 us on the GPU (3.0 TB/s).
+// ---------------------------------------------------------------------------
+template <typename T>
+__device__ inline void chunk_f32(uint4 u, float (&f)[8]) {
+  const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (__is_same(T, _Float16)) {
+      const kh2 h = __builtin_bit_cast(kh2, w[k]);
+      f[2 * k] = (float)h[0];
+      f[2 * k + 1] = (float)h[1];
+    } else {
+      f[2 * k] = __uint_as_float(w[k] << 16);
+      f[2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
+    }
+  }
+}
+
+// nv (1..8) 16-bit elements from element j0 of a row on, zero past them.  Any
+// 2-byte alignment (unaligned vector loads); a tail reads the 8 elements that
+// end with it, so nothing outside the row is touched.
+__device__ inline uint4 load_chunk(const uint16_t* row, int j0, int nv) {
+  uint4 u;
+  if (nv == 8) {
+    __builtin_memcpy(&u, row + j0, 16);
+    return u;
+  }
+  if (j0 >= 8) {
+    __builtin_memcpy(&u, row + j0 + nv - 8, 16);
+    const int drop = 16 * (8 - nv);                     // bits of the elements before j0
+    const uint64_t lo = (uint64_t)u.x | ((uint64_t)u.y << 32), hi = (uint64_t)u.z | ((uint64_t)u.w << 32);
+    const uint64_t l = drop < 64 ? (lo >> drop) | (hi << (64 - drop)) : hi >> (drop - 64);
+    const uint64_t h = drop < 64 ? hi >> drop : 0;
+    return make_uint4((uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32));
+  }
+  uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (e < nv) w[e >> 1] |= (uint32_t)row[j0 + e] << (16 * (e & 1));
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// the codes' integers ride in the low bits of y + 1.5 * 2^23 (+ a bias), the
+// addition rounding half to even as rint does
+constexpr float RINT_MAGIC = 12582912.f;
+__device__ inline uint32_t rint_bits(float y, float bias) { return __float_as_uint(y + (RINT_MAGIC + bias)); }
+
+// eight nibbles (codes + bias in 0..15) of the quotients y, already clamped
+__device__ inline uint32_t pack_nibbles(const float (&y)[8], float bias) {
+  uint32_t w = 0;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) w |= (rint_bits(y[e], bias) & 15u) << (4 * e);
+  return w;
+}
+
+// n bytes (1..8) of w to q, any alignment
+__device__ inline void store_bytes(uint8_t* q, uint64_t w, int n) {
+  if (n == 8) {
+    __builtin_memcpy(q, &w, 8);
+  } else if (n == 4) {
+    const uint32_t v = (uint32_t)w;
+    __builtin_memcpy(q, &v, 4);
+  } else {
+    for (int i = 0; i < n; ++i) q[i] = (uint8_t)(w >> (8 * i));
+  }
+}
+
+struct BlockPlan {
+  int nc, pp, nb;                       // chunks of a position's heads, positions per pass, blocks per batch
+  int ns;                               // scales per head (1, or 2 with a lower block)
+  uint16_t cstart[K_MAX_KV];            // first chunk of head h (0xffff past the last head)
+};
+
+// All heads of a run of positions per workgroup, so the packed source rows
+// ([B, T, sum of ranks]) are read as they lie: thread -> (position, 8-rank
+// chunk) of one pass, KC chunks per thread where a position has more than 256,
+// 8 / KC passes held in registers while the blocks' maxima meet in LDS.
+template <typename T, int KC, bool DENSE>
+__global__ __launch_bounds__(256) void append_block_kernel(const KAppendArgs a, const BlockPlan p) {
+  constexpr int U = 8 / KC;
+  extern __shared__ uint32_t sm[];
+  const int tid = threadIdx.x;
+  const int b = blockIdx.x / p.nb, t0 = (blockIdx.x - b * p.nb) * (p.pp * U);
+  const int P = p.pp * U;
+  const int nslot = a.H * p.ns * P;
+  float* const scale = (float*)sm;                       // [head][block][position]: maxima, then scales
+  float* const recip = scale + nslot;
+  const int pos = a.pos0_dev ? *a.pos0_dev : a.pos0;
+  const int pp = KC == 1 ? tid / p.nc : 0;
+  int head[KC], j0[KC], nv[KC];
+  uint4 x[KC][U];
+#pragma unroll
+  for (int k = 0; k < KC; ++k) {
+    const int c = (KC == 1 ? tid - pp * p.nc : tid) + 256 * k;
+    int h = -1;
+#pragma unroll
+    for (int i = 0; i < K_MAX_KV; ++i) h += c >= p.cstart[i];
+    head[k] = h;
+    j0[k] = 8 * (c - p.cstart[h]);
+    nv[k] = c < p.nc && pp < p.pp ? min(8, a.rank[h] - j0[k]) : 0;
+    const uint16_t* src = (const uint16_t*)a.src + b * a.src_sb + a.src_off[h];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (nv[k] > 0) x[k][u] = load_chunk(src + (int64_t)min(t0 + u * p.pp + pp, a.T - 1) * a.src_st, j0[k], nv[k]);
+  }
+  if (a.err != nullptr)
+    for (int i = t0 + tid; i < min(t0 + P, a.T); i += 256)
+      if (pos + i < 0 || pos + i >= a.cap) *a.err = 1;
+  if constexpr (DENSE) {
+#pragma unroll
+    for (int k = 0; k < KC; ++k)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int t = t0 + u * p.pp + pp, s = pos + t;
+        if (nv[k] <= 0 || t >= a.T || s < 0 || s >= a.cap) continue;
+        uint16_t* d = (uint16_t*)a.data + b * a.stride_b + a.off[head[k]] + (int64_t)s * a.pitch[head[k]] + j0[k];
+        if (nv[k] == 8) {
+          __builtin_memcpy(d, &x[k][u], 16);
+        } else {
+          const uint32_t w[4] = {x[k][u].x, x[k][u].y, x[k][u].z, x[k][u].w};
+#pragma unroll
+          for (int e = 0; e < 7; ++e)
+            if (e < nv[k]) d[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+        }
+      }
+    return;
+  }
+  for (int i = tid; i < nslot; i += 256) sm[i] = 0;
+  __syncthreads();
+  int slot[KC];
+#pragma unroll
+  for (int k = 0; k < KC; ++k) {
+    slot[k] = (head[k] * p.ns + (j0[k] >= a.split)) * P + pp;
+    if (nv[k] <= 0) continue;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float f[8], m = 0.f;
+      chunk_f32<T>(x[k][u], f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(f[e]));
+      atomicMax(&sm[slot[k] + u * p.pp], __float_as_uint(m));   // non-negative floats order as their bits
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < nslot; i += 256) {
+    const int seg = i / P, t = t0 + (i - seg * P), s = pos + t;
+    const int h = p.ns == 2 ? seg >> 1 : seg;
+    const bool lower = p.ns == 2 && (seg & 1);
+    const _Float16 s16 = fp16_scale(scale[i], !lower && a.a_int8 ? 127.f : 7.f);
+    scale[i] = (float)s16;
+    recip[i] = __fdiv_rn(1.f, (float)s16);
+    if (t >= a.T || s < 0 || s >= a.cap || (lower && a.rank[h] <= a.split)) continue;
+    uint16_t* sp = lower ? (uint16_t*)a.scale2 + b * a.sc2_sb + h * a.sc2_sh + (int64_t)s * a.sc2_ss
+                         : (uint16_t*)a.scale + b * a.sc_sb + h * a.sc_sh + (int64_t)s * a.sc_ss;
+    *sp = __builtin_bit_cast(uint16_t, s16);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < KC; ++k) {
+    if (nv[k] <= 0) continue;
+    const int h = head[k];
+    const bool lower = j0[k] >= a.split, i8 = !lower && a.a_int8;
+    const int jb = lower ? j0[k] - a.split : j0[k];
+    uint8_t* q = (lower ? (uint8_t*)a.data2 + b * a.stride2_b + a.off2[h] : (uint8_t*)a.data + b * a.stride_b + a.off[h]) +
+                 (i8 ? jb : jb >> 1);
+    const int64_t pitch = lower ? a.pitch2[h] : a.pitch[h];
+    const float lo = i8 ? -127.f : -8.f, hi = i8 ? 127.f : 7.f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int t = t0 + u * p.pp + pp, s = pos + t;
+      if (t >= a.T || s < 0 || s >= a.cap) continue;
+      const float sc = scale[slot[k] + u * p.pp], rc = recip[slot[k] + u * p.pp];
+      float f[8];
+      chunk_f32<T>(x[k][u], f);
+      if (sc < INFINITY) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float y = f[e] * rc;
+          f[e] = fmaf(fmaf(-y, sc, f[e]), rc, y);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = __fdiv_rn(f[e], sc);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = fminf(fmaxf(f[e], lo), hi);
+      uint8_t* d = q + (int64_t)s * pitch;
+      if (i8) {
+        uint32_t w[2];
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          const uint32_t e01 = __builtin_amdgcn_perm(rint_bits(f[4 * v + 1], 0.f), rint_bits(f[4 * v], 0.f), 0x0C0C0400u);
+          const uint32_t e23 = __builtin_amdgcn_perm(rint_bits(f[4 * v + 3], 0.f), rint_bits(f[4 * v + 2], 0.f), 0x04000C0Cu);
+          w[v] = e01 | e23;
+        }
+        store_bytes(d, (uint64_t)w[0] | ((uint64_t)w[1] << 32), nv[k]);
+      } else {
+        store_bytes(d, pack_nibbles(f, 8.f), (nv[k] + 1) >> 1);   // past an odd rank: 0 / s, nibble 8
+      }
+    }
+  }
+}
+
+// Group-64 V rows: thread -> 8-rank chunk, a group's eight threads reduce its
+// minimum and maximum among themselves; U chunks in flight per thread.
+template <typename T>
+__global__ __launch_bounds__(256) void append_g64_kernel(const VAppendArgs a, int nb) {
+  constexpr int U = 4;
+  const int b = blockIdx.x / nb;
+  const uint32_t first = (uint32_t)(blockIdx.x - b * nb) * (256 * U) + threadIdx.x;
+  const uint32_t ncg = (uint32_t)((a.R + 63) >> 6) * 8, total = ncg * (uint32_t)a.T;
+  const int pos = a.pos0_dev ? *a.pos0_dev : a.pos0;
+  uint4 x[U];
+  int tt[U], j0[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint32_t i = min(first + 256 * u, total - 8 + (threadIdx.x & 7));   // past the end: the last group again
+    const uint32_t t = i / ncg;
+    tt[u] = (int)t;
+    j0[u] = 8 * (int)(i - t * ncg);
+    const int nv = min(8, a.R - j0[u]);
+    x[u] = make_uint4(0, 0, 0, 0);
+    if (nv > 0) x[u] = load_chunk((const uint16_t*)a.src + b * a.src_sb + (int64_t)t * a.src_st, j0[u], nv);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int nv = min(8, a.R - j0[u]), s = pos + tt[u];
+    float f[8], lo = INFINITY, hi = -INFINITY;
+    chunk_f32<T>(x[u], f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      lo = e < nv ? fminf(lo, f[e]) : lo;
+      hi = e < nv ? fmaxf(hi, f[e]) : hi;
+    }
+#pragma unroll
+    for (int o = 4; o >= 1; o >>= 1) {
+      lo = fminf(lo, __shfl_xor(lo, o, 8));
+      hi = fmaxf(hi, __shfl_xor(hi, o, 8));
+    }
+    const _Float16 z16 = (_Float16)lo;
+    const float z = (float)z16;
+    _Float16 s16 = (_Float16)__fdiv_rn(hi - z, 15.f);
+    if ((float)s16 == 0.f) s16 = (_Float16)1.0f;
+    const float sc = (float)s16;
+    if (s < 0 || s >= a.cap) {                        // only a run-time position can land here
+      if (a.err != nullptr) *a.err = 1;
+      continue;
+    }
+    if (first + 256 * u >= total) continue;
+    if ((threadIdx.x & 7) == 0) {
+      const int64_t o = b * a.sc_sb + (int64_t)s * a.sc_ss + (j0[u] >> 6);
+      ((uint16_t*)a.scale)[o] = __builtin_bit_cast(uint16_t, s16);
+      ((uint16_t*)a.zero)[o] = __builtin_bit_cast(uint16_t, z16);
+    }
+    if (nv <= 0) continue;
+    if (fabsf(sc) < INFINITY) {
+      const float rc = __fdiv_rn(1.f, sc);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float d = f[e] - z;
+        float y = d * rc;
+        y = fmaf(fmaf(-y, sc, d), rc, y);
+        f[e] = fmaf(fmaf(-y, sc, d), rc, y);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = __fdiv_rn(f[e] - z, sc);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = e < nv ? fminf(fmaxf(f[e], 0.f), 15.f) : 0.f;
+    store_bytes((uint8_t*)a.data + b * a.stride_b + (int64_t)s * a.stride_s + (j0[u] >> 1), pack_nibbles(f, 0.f),
+                (nv + 1) >> 1);
+  }
+}
+
+template <typename T, int KC>
+static void launch_block_t(const KAppendArgs& a, const BlockPlan& p, hipStream_t st) {
+  const dim3 grid((unsigned)(a.B * p.nb));
+  const size_t lds = (size_t)a.H * p.ns * p.pp * (8 / KC) * 8;
+  if (a.fmt == STARKV_FMT_DENSE) hipLaunchKernelGGL((append_block_kernel<T, KC, true>), grid, dim3(256), 0, st, a, p);
+  else hipLaunchKernelGGL((append_block_kernel<T, KC, false>), grid, dim3(256), lds, st, a, p);
+}
+
+static void launch_block(const KAppendArgs& a, int dtype, hipStream_t st) {
+  BlockPlan p = {};
+  bool two = false;
+  for (int h = 0; h < K_MAX_KV; ++h) {
+    p.cstart[h] = h < a.H ? (uint16_t)p.nc : (uint16_t)0xffff;
+    if (h >= a.H) continue;
+    p.nc += (a.rank[h] + 7) / 8;
+    two |= a.rank[h] > a.split;
+  }
+  p.ns = two ? 2 : 1;
+  const int kc = p.nc <= 256 ? 1 : p.nc <= 512 ? 2 : 4;   // at most 64 * 16 (K) or 8192 / 8 (V) chunks
+  p.pp = kc == 1 ? 256 / p.nc : 1;
+  p.nb = (int)ceil_div(a.T, p.pp * (8 / kc));
+  const bool h = dtype == STARKV_F16;
+  if (kc == 1) h ? launch_block_t<_Float16, 1>(a, p, st) : launch_block_t<__bf16, 1>(a, p, st);
+  else if (kc == 2) h ? launch_block_t<_Float16, 2>(a, p, st) : launch_block_t<__bf16, 2>(a, p, st);
+  else h ? launch_block_t<_Float16, 4>(a, p, st) : launch_block_t<__bf16, 4>(a, p, st);
+}
+
+static void launch_v_rows(const VAppendArgs& a, int dtype, hipStream_t st) {
+  if (a.vq == VQ_G64) {
+    const int nb = (int)ceil_div((int64_t)a.T * ceil_div(a.R, 64) * 8, 256 * 4);
+    const dim3 grid((unsigned)(a.B * nb));
+    if (dtype == STARKV_F16) hipLaunchKernelGGL(append_g64_kernel<_Float16>, grid, dim3(256), 0, st, a, nb);
+    else hipLaunchKernelGGL(append_g64_kernel<__bf16>, grid, dim3(256), 0, st, a, nb);
+    return;
+  }
+  // a dense or per-token block row is one head whose scales step by sc_ss
+  KAppendArgs k = {};
+  k.src = a.src; k.src_sb = a.src_sb; k.src_st = a.src_st;
+  k.B = a.B; k.H = 1; k.T = a.T; k.pos0 = a.pos0; k.cap = a.cap; k.pos0_dev = a.pos0_dev; k.err = a.err;
+  k.fmt = a.vq == VQ_DENSE ? STARKV_FMT_DENSE : STARKV_FMT_INT4_REF;
+  k.data = a.data; k.stride_b = a.stride_b; k.pitch[0] = a.stride_s;
+  k.scale = a.scale; k.sc_sb = a.sc_sb; k.sc_ss = a.sc_ss;
+  k.split = a.vq == VQ_DENSE ? a.R : a.split; k.a_int8 = a.a_int8;
+  k.data2 = a.data2; k.stride2_b = a.stride2_b; k.pitch2[0] = a.stride2_s;
+  k.scale2 = a.scale2; k.sc2_sb = a.sc2_sb; k.sc2_ss = a.sc2_ss;
+  k.rank[0] = a.R;
+  launch_block(k, dtype, st);
+}
+
+// The chunked kernels take over where their ~10 us of fixed time (two launches,
+// each a chain of loads, maxima and divisions) pays: from 16384 rows on
+// (positions x heads, or x 64-rank groups of V), 32768 unquantised.  Measured,
+// K and V written together, row-per-wave against chunked, us: 32 heads, int8 /
+// group-64: 512 positions 12.6 / 13.1, 2048 43.7 / 16.2, 16384 310 / 51;
+// dense: 512 8.8 / 10.4, 1024 12.5 / 11.1, 16384 142 / 39.  8 heads, int8 /
+// group-64: 2048 positions 13.5 / 14.2, 16384 93 / 24; dense: 2048 7.0 / 10.5,
+// 16384 41 / 20.  A workgroup holds 8 or more positions of one batch: runs of
+// fewer than 16 stay with the row-per-wave kernels.
+static bool many_rows(int B, int T, int per_pos, bool dense) {
+  return T >= 16 && (int64_t)B * T * per_pos >= (dense ? 32768 : 16384);
+}
+static bool many_rows(const KAppendArgs& a) { return many_rows(a.B, a.T, a.H, a.fmt == STARKV_FMT_DENSE); }
+static bool many_rows(const VAppendArgs& a) { return many_rows(a.B, a.T, (int)ceil_div(a.R, 64), a.vq == VQ_DENSE); }
+
 int launch_step_append(const StepAppendArgs& a0, int dtype, hipStream_t st) {
   StepAppendArgs a = a0;
+  if (many_rows(a.k)) {
+    launch_block(a.k, dtype, st);
+    launch_v_rows(a.v, dtype, st);
+    if (a.has_rope) return launch_rope_apply(a.r, dtype, st);
+    return (int)hipGetLastError();
+  }
   a.v.gw = a.v.vq == VQ_G64 ? (int)ceil_div(a.v.R, 64) : 1;
   a.nbk = ceil_div((int64_t)a.k.B * a.k.H * a.k.T, 4);
   a.nbv = ceil_div((int64_t)a.v.B * a.v.T * a.v.gw, 4);
@@ -194,6 +556,10 @@ int launch_step_append(const StepAppendArgs& a0, int dtype, hipStream_t st) {
 int launch_k_append(const KAppendArgs& a, int dtype, hipStream_t st) {
   const int64_t rows = (int64_t)a.B * a.H * a.T;
   if (rows == 0) return 0;
+  if (many_rows(a)) {
+    launch_block(a, dtype, st);
+    return (int)hipGetLastError();
+  }
   const dim3 grid((unsigned)ceil_div(rows, 4));
   if (dtype == STARKV_F16) hipLaunchKernelGGL(k_append_kernel<_Float16>, grid, dim3(256), 0, st, a);
   else hipLaunchKernelGGL(k_append_kernel<__bf16>, grid, dim3(256), 0, st, a);
@@ -203,6 +569,10 @@ int launch_k_append(const KAppendArgs& a, int dtype, hipStream_t st) {
 int launch_v_append(const VAppendArgs& a, int dtype, hipStream_t st) {
   const int64_t rows = (int64_t)a.B * a.T;
   if (rows == 0) return 0;
+  if (many_rows(a)) {
+    launch_v_rows(a, dtype, st);
+    return (int)hipGetLastError();
+  }
   VAppendArgs r = a;
   r.gw = a.vq == VQ_G64 ? (int)ceil_div(a.R, 64) : 1;
   const dim3 grid((unsigned)ceil_div(rows * r.gw, 4));
