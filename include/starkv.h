@@ -111,9 +111,9 @@ int starkv_rope_apply(const starkv_rope_apply_desc* d, void* stream);
  * bk + bk_head_offset[h] + j*bk_row_stride, 128 contiguous elements.
  *
  * Any rank 1..128 and any row layout in every format.  Dense rows that the
- * streaming K-logit kernels cannot read (a rank that is not a multiple of 8,
- * or rows not 16-byte aligned) are copied by starkv_k_logits into its
- * workspace first; quantised rows of any byte alignment are read as aligned
+ * streaming K-logit kernels cannot read (neither contiguous nor 16-byte
+ * aligned with a rank that is a multiple of 8) are copied by starkv_k_logits
+ * into its workspace first; quantised rows of any byte alignment are read as aligned
  * words joined in registers.
  * Quantised K (offsets and strides of data/data2 in bytes; every value
  * dequantised to fp16 before use, as the reference's
@@ -170,7 +170,8 @@ typedef struct {
  * streamed in place (dense: ranks multiples of 8 on 16-byte aligned rows;
  * int8 or the split format: always), else the size of a padded copy of the
  * dense K latent ([B][Hkv][S] rows of round_up(r, 8) elements, 16-byte pitch)
- * that the call writes before the logits.
+ * that the call writes before the logits unless every head's rows are
+ * contiguous (the kernels then stage them as they lie).
  * ------------------------------------------------------------------- */
 typedef struct {
   int batch, n_q_heads, head_dim, seq_len;

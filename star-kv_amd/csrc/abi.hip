@@ -161,17 +161,58 @@ bool k_quant_aligned(const starkv_klatent& k) {
   return true;
 }
 
+// Dense head whose rows the streaming kernels stage in whole 16-byte pieces:
+// rank a multiple of 8 (or a padded copy), rows 16-byte aligned in every batch.
+bool ws_rows16(const starkv_klatent& k, int h, int xe, bool padded) {
+  return al(k.data, 16) && al64(k.stride_b * xe, 16) && (k.rank[h] % 8 == 0 || padded) &&
+         al64(k.head_offset[h] * xe, 16) && al64(k.pos_stride[h] * xe, 16);
+}
+// Other dense heads with contiguous rows are staged as runs of bytes (see
+// KArgs::klin) by the same kernels instead of being copied into aligned rows
+// or read element by element by the register-streaming kernel (8 KV heads of
+// rank 102, groups of 4, B1 S65536: 83 us a call with the copy, 55 us without;
+// 32 heads of odd ranks, B3 S5003: the decode call 148 against 111 us, its K
+// logits 69 us before).  Below 8 ranks a row holds no whole chunk.  The grouped-query kernel stages either
+// all heads of a launch so or none, and its DMA slots hold two linear heads of
+// up to 127 ranks.
+bool ws_linear(const starkv_klatent& k, int h, int gs) {
+  return k.format == STARKV_FMT_DENSE && k.pos_stride[h] == k.rank[h] && k.rank[h] >= 8 && k.rank[h] <= (gs > 1 ? 127 : 128) &&
+         al(k.data, 2);
+}
+// The heads of a dense launch staged as runs of bytes; ok: every head is
+// staged in one form or the other.
+struct LinPlan {
+  bool ok;
+  uint64_t mask;
+};
+LinPlan lin_plan(const starkv_klatent& k, int gs, int xe, bool padded) {
+  LinPlan p = {true, 0};
+  bool all = true;
+  for (int h = 0; h < k.n_kv_heads; ++h) {
+    const bool l = ws_linear(k, h, gs);
+    all = all && l;
+    if (ws_rows16(k, h, xe, padded)) continue;
+    if (!l) return {false, 0};
+    p.mask |= (uint64_t)1 << h;
+  }
+  if (p.mask && gs > 1) {
+    if (!all) return {false, 0};
+    for (int h = 0; h < k.n_kv_heads; ++h) p.mask |= (uint64_t)1 << h;
+  }
+  return p;
+}
+
 // Warp-specialised K-logit kernel: dense latents with 16-byte aligned rows
-// (ranks a multiple of 8), or int8 latents with one scale per (b, h, s) whose
+// (ranks a multiple of 8) or contiguous ones (ws_linear), or int8 latents with one scale per (b, h, s) whose
 // rows start on 16-byte boundaries (pitch a multiple of 16 bytes, so the 16-byte
 // DMA pieces never straddle rows); q and B_k are read element-wise there.
 // padded: dense rows hold round_up(r, 8) elements, zero past r (the K-logit
 // entry's repacked copy), so a rank need not be a multiple of 8.
-bool k_ws(const starkv_klatent& k, int dtype, int S, bool padded = false) {
+bool k_ws(const starkv_klatent& k, int gs, int dtype, int S, bool padded = false) {
   const bool i8 = k.format == STARKV_FMT_INT8_SYM;
   if (k.format != STARKV_FMT_DENSE && !i8) return false;
   const int xe = i8 ? 1 : esize(dtype);
-  if (!al(k.data, 16) || !al64(k.stride_b * xe, 16)) return false;
+  if (i8 && (!al(k.data, 16) || !al64(k.stride_b * xe, 16))) return false;
   // int8: the scales of a tile are staged in 16-byte pieces (8 positions), so
   // each (b, h) scale row is read up to position round_up(S, 8) - 1, inside
   // its pitch
@@ -179,11 +220,10 @@ bool k_ws(const starkv_klatent& k, int dtype, int S, bool padded = false) {
              k.scale_stride_h < round_up(S, 8)))
     return false;
   for (int h = 0; h < k.n_kv_heads; ++h) {
-    if (k.rank[h] % 8 && !(padded && !i8)) return false;
-    if (!al64(k.head_offset[h] * xe, 16) || !al64(k.pos_stride[h] * xe, 16)) return false;
+    if (i8 && (k.rank[h] % 8 || !al64(k.head_offset[h], 16) || !al64(k.pos_stride[h], 16))) return false;
     if ((int64_t)TILE * k.pos_stride[h] * xe >= ((int64_t)1 << 31)) return false;   // 32-bit per-tile DMA step
   }
-  return true;
+  return i8 || lin_plan(k, gs, xe, padded).ok;
 }
 
 // 16-byte LDS chunks of one 32-position tile row of a head in that kernel
@@ -305,7 +345,7 @@ static bool ws_balance(const starkv_klatent& k, int Hq, int unit, int nw, int ca
 // 4 waves (4-item waves).
 int build_k_plan(const starkv_klatent& k, int Hq, int gs, int dtype, int S, KArgs& a, KPlan& plan,
                  bool padded = false) {
-  const bool ws = k_ws(k, dtype, S, padded);
+  const bool ws = k_ws(k, gs, dtype, S, padded);
   const int unit = 32;                        // ranks per item
   struct QH { int qh, kv, ni; };              // ni: items of the head
   std::vector<QH> heads;
@@ -428,6 +468,7 @@ int build_k_plan(const starkv_klatent& k, int Hq, int gs, int dtype, int S, KArg
   }
   a.gqa = gqa;
   a.gs = gs;
+  a.klin = ws && k.format == STARKV_FMT_DENSE ? lin_plan(k, gs, esize(dtype), padded).mask : 0;
   for (int h = 0; h < K_MAX_KV; ++h) a.krank[h] = (int16_t)(h < k.n_kv_heads ? k.rank[h] : 0);
   const bool two = k.format == STARKV_FMT_INT4_REF && k.split > 0;
   a.ksplit = two ? k.split : 128;
@@ -461,7 +502,7 @@ int build_k_plan(const starkv_klatent& k, int Hq, int gs, int dtype, int S, KArg
           const int kv = (it >> 8) & 0xff;
           if (!((it >> 27) & 1) || seen[kv]) continue;
           seen[kv] = true;
-          chunks += 32 * ws_row_chunks(k, kv);
+          chunks += (a.klin >> kv) & 1 ? (gqa ? (int)round_up(lin_chunks(k.rank[kv]), 64) : lin_chunks(k.rank[kv])) : 32 * ws_row_chunks(k, kv);
         }
       max_chunks = std::max(max_chunks, chunks);
     }
@@ -839,26 +880,33 @@ int starkv_rope_build(const float* inv_freq_host, float attention_scaling, int m
 }
 
 // Dense K whose rows the warp-specialised and grouped-query K-logit kernels
-// cannot stream (a rank not a multiple of 8, or rows not 16-byte aligned: the
-// reference abx benchmark's 102 ranks per KV head, abx_rope_batched.py:274-280,
-// leaves 204-byte rows) is first copied into the workspace as rows of
-// round_up(r, 8) elements, zero past r, one 16-byte pitch for all heads
-// ([B][Hkv][S][pitch]); the kernels then read that copy.
+// cannot stream (rows that are neither 16-byte aligned multiples of 8 ranks
+// nor contiguous, or fewer than 8 ranks) is first copied into the workspace as
+// rows of round_up(r, 8) elements, zero past r, one 16-byte pitch for all
+// heads ([B][Hkv][S][pitch]); the kernels then read that copy.  Every latent
+// without aligned rows of whole 8-rank chunks asks for the copy's workspace,
+// whether its kernel uses it or not.
 struct KRepack {
-  bool on = false;
+  bool need = false;          // ask for the workspace
+  bool on = false;            // make the copy
   int pitch = 0;              // bytes
   size_t bytes = 0;
 };
 
-KRepack k_repack_plan(const starkv_klatent& k, int dtype, int B, int S) {
+KRepack k_repack_plan(const starkv_klatent& k, int gs, int dtype, int B, int S) {
   KRepack r;
-  if (k.format != STARKV_FMT_DENSE || k_ws(k, dtype, S)) return r;
+  if (k.format != STARKV_FMT_DENSE) return r;
+  const bool ws = k_ws(k, gs, dtype, S);
+  bool rows16 = ws;
+  for (int h = 0; h < k.n_kv_heads; ++h) rows16 = rows16 && ws_rows16(k, h, esize(dtype), false);
+  if (rows16) return r;
   int rmax = 8;
   for (int h = 0; h < k.n_kv_heads; ++h) rmax = std::max(rmax, k.rank[h]);
   r.pitch = (int)round_up((int64_t)round_up(rmax, 8) * esize(dtype), 16);
   if ((int64_t)TILE * r.pitch >= ((int64_t)1 << 31)) return r;
   r.bytes = a256((size_t)B * k.n_kv_heads * S * r.pitch);
-  r.on = true;
+  r.need = true;
+  r.on = !ws;
   return r;
 }
 
@@ -866,7 +914,7 @@ size_t starkv_k_logits_workspace_bytes(const starkv_klogits_desc* d) {
   int gs = 0;
   if (!d || d->batch < 1 || d->seq_len < 1 || d->seq_len > MAX_S || validate_klatent(d->k, d->n_q_heads, d->dtype, &gs))
     return 0;
-  return k_repack_plan(d->k, d->dtype, d->batch, d->seq_len).bytes;
+  return k_repack_plan(d->k, gs, d->dtype, d->batch, d->seq_len).bytes;
 }
 
 int starkv_k_logits(const starkv_klogits_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
@@ -878,12 +926,14 @@ int starkv_k_logits(const starkv_klogits_desc* d, void* workspace, size_t worksp
   if (d->seq_len > d->rope_max_positions) return STARKV_ERR_SHAPE;
   if (d->out_dtype != STARKV_F32 && d->out_dtype != STARKV_F16 && d->out_dtype != STARKV_BF16) return STARKV_ERR_DTYPE;
   if ((st = check_mask(d->mask, d->mask_dtype))) return st;
-  const KRepack rp = k_repack_plan(d->k, d->dtype, d->batch, d->seq_len);
+  const KRepack rp = k_repack_plan(d->k, gs, d->dtype, d->batch, d->seq_len);
   starkv_klatent k = d->k;
   int64_t rp_hoff[K_MAX_KV], rp_pstr[K_MAX_KV];   // the repacked copy's head offsets and row pitches
-  if (rp.on) {
+  if (rp.need) {
     if (!workspace || workspace_bytes < rp.bytes) return STARKV_ERR_WORKSPACE;
     if (!al(workspace, 256)) return STARKV_ERR_ALIGN;
+  }
+  if (rp.on) {
     const int H = k.n_kv_heads, S = d->seq_len, xe = esize(d->dtype);
     RepackArgs ra = {};
     ra.src = (const uint8_t*)k.data; ra.src_sb = k.stride_b * xe;

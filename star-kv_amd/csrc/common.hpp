@@ -75,7 +75,23 @@ struct KArgs {
   // once per KV head; item 0 of consumer wave w = item_pack(kv * gs, kv, dim half, 0, 1)
   int gqa, gs;
   int16_t krank[K_MAX_KV];
+  // dense heads whose tiles are staged as one run of bytes (bit kv; ws_linear
+  // in abi.hip): contiguous rows of any rank and alignment
+  uint64_t klin;
 };
+
+// A linear head's tile is 32 rows of 2r contiguous bytes: 64r bytes from the
+// 16-byte piece that holds its first one, at most 4r + 1 pieces.  Rows lie at
+// any 2-byte offset in LDS (unaligned reads).  A lane's chunk of 8 ranks that
+// would pass the rank starts at rank r - 8 instead, so every element read is
+// the row's own; the operand it meets holds zeros for the ranks the chunk
+// before covers already.  lin_rank: the rank of element i of chunk c, or -1.
+__host__ __device__ inline int lin_chunks(int r) { return 4 * r + 1; }
+__device__ inline int lin_start(int r, int c) { return min(8 * c, r - 8); }
+__device__ inline int lin_rank(int r, int c, int i) {
+  const int j = lin_start(r, c) + i;
+  return 8 * c < r && j >= 8 * c ? j : -1;
+}
 constexpr int K1_GQ_CARRY_BYTES = 2 * 2 * 64 * 4 * 4;          // GQA: dim-half partial logits, 2 tiles x 2 heads
 constexpr int K1_GQ_RING_BYTES = 81920 - K1_GQ_CARRY_BYTES;    // its LDS ring (two workgroups per CU)
 

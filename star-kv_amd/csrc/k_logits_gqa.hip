@@ -92,7 +92,8 @@ __device__ inline floatx16 gq_mfma(typename GqVec<XT>::T a, typename GqVec<XT>::
 }
 
 // this wave's share of every tile's DMA: instructions m = wave + 4k
-struct GqDma {
+template <bool LIN> struct GqDma;
+template <> struct GqDma<false> {
   const char* base[GQ_MAXK];   // lane address at tile0
   uint32_t lstep[GQ_MAXK];     // bytes per tile (< 2^31, checked on the host)
   int rowp[GQ_MAXK];           // latent: the lane's row in a tile; RoPE operand: -2^30 (never clamped)
@@ -124,6 +125,41 @@ struct GqDma {
   }
 };
 
+// The same for linear heads (KArgs::klin): each head's run of bytes is staged
+// in whole 1 KB instructions of its own, so everything but the lane's 16-byte
+// slot is uniform (per-lane addresses of runs that share instructions, as
+// above, spilled 19 registers).  Pieces past the one that holds the last row's
+// last byte re-read it; those past the tile read the next tile's bytes.
+template <> struct GqDma<true> {
+  const char* base[GQ_MAXH];   // the 16-byte piece that holds each head's first byte of tile0
+  int64_t lim[GQ_MAXH];        // offset from there of the piece that holds the last row's last byte
+  uint32_t step[GQ_MAXH];      // bytes per tile
+  const char* rope;            // the RoPE operand of tile0
+  int n0, nx;                  // instructions of the first head, of both
+  int wave, cnt;
+  uint32_t slot;               // 16 * lane
+  uint32_t ring;
+  int stage, nst, tile0;
+
+  __device__ inline void issue(int i) const {
+    const uint32_t lb = ring + (uint32_t)((i % nst) * stage);
+#pragma unroll
+    for (int k = 0; k < GQ_MAXK; ++k) {
+      const int m = wave + GQ_WAVES * k;
+      if (k >= cnt) break;
+      if (m < nx) {
+        const bool h = m >= n0;
+        const int64_t off = (int64_t)i * (h ? step[1] : step[0]);
+        const int64_t rest = (h ? lim[1] : lim[0]) - off;
+        const uint32_t at = min(slot + (uint32_t)(h ? m - n0 : m) * 1024u, (uint32_t)min(rest, (int64_t)1 << 30));
+        gq_dma((h ? base[1] : base[0]) + off + at, lb + (uint32_t)m * 1024u);
+      } else {
+        gq_dma(rope + (int64_t)i * 8192 + (m - nx) * 1024 + slot, lb + (uint32_t)(stage - 8192 + (m - nx) * 1024));
+      }
+    }
+  }
+};
+
 // the workgroup's KV heads and where their rows sit in a stage
 struct GqHeads {
   int hkv[GQ_MAXH], hrank[GQ_MAXH], hoff[GQ_MAXH];
@@ -138,12 +174,13 @@ struct GqHeads {
 // which the compiler waits for with counts that do not see the DMA, drain
 // the ring once per tile; the unmasked kernel issues no waited-for load in
 // its loop).
-template <typename XT, int OUTK, int NK, bool MASKED>
-__device__ __attribute__((always_inline)) inline void gq_consume(const KArgs& a, const GqHeads& H, const GqDma& d,
+template <typename XT, int OUTK, int NK, bool MASKED, bool LIN>
+__device__ __attribute__((always_inline)) inline void gq_consume(const KArgs& a, const GqHeads& H, const GqDma<LIN>& d,
                                                                   char* ring, float (*carry)[GQ_MAXH][64][4],
                                                                   int slot, int p, int kv, int b, int chunk, int ntl,
                                                                   int ahead) {
   typedef typename GqVec<XT>::T XV;
+  typedef XV __attribute__((aligned(LIN ? 2 : 16))) XU;
   const int lane = threadIdx.x & 63, t = lane & 31, hh = lane >> 5;
   const int gs = a.gs, S = a.S, tile0 = d.tile0, stage = d.stage, nst = d.nst;
   const int r = H.hrank[slot], hb = H.hoff[slot], n16 = (r + 7) >> 3;   // chunks of a row (padded rows past r)
@@ -175,8 +212,9 @@ __device__ __attribute__((always_inline)) inline void gq_consume(const KArgs& a,
         XV v;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const int rk = 16 * kk + 8 * hh + i;
-          v[i] = rk < r ? bk[(int64_t)rk * a.bk_rs + dim] : (XT)0.f;
+          // (all chunks but those of the last two K-steps lie below the rank)
+          const int rk = LIN && kk >= NK - 2 ? lin_rank(r, 2 * kk + hh, i) : 16 * kk + 8 * hh + i;
+          v[i] = rk >= 0 && rk < r ? bk[(int64_t)rk * a.bk_rs + dim] : (XT)0.f;
         }
         bt[mi][kk] = v;
       }
@@ -211,6 +249,11 @@ __device__ __attribute__((always_inline)) inline void gq_consume(const KArgs& a,
   for (int kk = 0; kk < NK; ++kk) {
     const int c = min(2 * kk + hh < n16 ? 2 * kk + hh : 2 * kk, n16 - 1);
     xo[kk] = (hb + t * n16 + (c + gq_shift(t, n16)) % n16) * 16;
+    if constexpr (LIN) {
+      const char* head = (const char*)a.x + (b * a.x_sb + a.xoff[kv]) * 2;
+      const int row0 = hb * 16 + (int)((uintptr_t)head & 15) + t * 2 * r;
+      xo[kk] = kk < NK - 2 ? row0 + 16 * hh + 32 * kk : row0 + 2 * lin_start(r, c);
+    }
   }
   // query rows h < gs <= 8 are accumulator entries v = h % 4 of lane half h / 4
   // operands in before the ring fills: the compiler's waits for them, which
@@ -279,7 +322,7 @@ __device__ __attribute__((always_inline)) inline void gq_consume(const KArgs& a,
     auto tile_logits = [&](float ks, float sum[4]) __attribute__((always_inline)) {
       XV xb[NK];
 #pragma unroll
-      for (int kk = 0; kk < NK; ++kk) xb[kk] = *(const XV*)(st + xo[kk]);
+      for (int kk = 0; kk < NK; ++kk) xb[kk] = *(const XU*)(st + xo[kk]);
       half8 T4[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g) T4[g] = *(const half8*)(st + stage - 8192 + ((4 * p + g) * 64 + lane) * 16);
@@ -364,7 +407,8 @@ __device__ __attribute__((always_inline)) inline void gq_consume(const KArgs& a,
 }
 
 // OUTK: 0 = fp32 logits + chunk maxima, 1 = fp16 logits, 2 = bf16 logits
-template <typename XT, int OUTK, bool MASKED>
+// LIN: every head's tiles staged as runs of bytes (KArgs::klin)
+template <typename XT, int OUTK, bool MASKED, bool LIN>
 __global__ __launch_bounds__(GQ_WAVES * 64, 2) void k_logits_gqa_kernel(const KArgs a) {
   __shared__ __attribute__((aligned(16))) char ring[GQ_RING];          // a.ws_nst stages of a.ws_stage bytes
   __shared__ float carry[2][GQ_MAXH][64][4];                           // p = 0 partial logits, by tile parity
@@ -391,7 +435,7 @@ __global__ __launch_bounds__(GQ_WAVES * 64, 2) void k_logits_gqa_kernel(const KA
     H.hkv[k] = item_kv(itm);
     H.hrank[k] = a.krank[H.hkv[k]];
     H.hoff[k] = H.tot;
-    H.tot += 32 * ((H.hrank[k] + 7) >> 3);
+    H.tot += LIN ? (lin_chunks(H.hrank[k]) + 63) & ~63 : 32 * ((H.hrank[k] + 7) >> 3);
   }
   // stage: latent chunks [0, 64 * nX), the RoPE operand in the last 8 KB
   const int nX = (H.tot + 63) / 64, stage = a.ws_stage, nst = a.ws_nst;
@@ -399,8 +443,27 @@ __global__ __launch_bounds__(GQ_WAVES * 64, 2) void k_logits_gqa_kernel(const KA
   const int ahead = nst - 1;     // stage of tile i - 1 (its reads ended at barrier i) takes tile i + ahead
 
   // ---- this wave's DMA share
-  GqDma d;
-  {
+  GqDma<LIN> d;
+  if constexpr (LIN) {
+#pragma unroll
+    for (int k = 0; k < GQ_MAXH; ++k) {
+      const int hk = H.hkv[k], r = H.hrank[k];
+      const char* head = (const char*)a.x + (b * a.x_sb + a.xoff[hk]) * 2;
+      const int mis = (int)((uintptr_t)head & 15);
+      const int64_t first = (int64_t)tile0 * 64 * r;
+      d.base[k] = head - mis + first;
+      d.lim[k] = ((mis + (int64_t)2 * r * S - 1) & ~(int64_t)15) - first;
+      d.step[k] = (uint32_t)(64 * r);
+    }
+    d.rope = (const char*)a.rope + (int64_t)tile0 * 8192;
+    d.n0 = min(H.hoff[1], H.tot) >> 6;
+    d.nx = nX;
+    d.wave = wave;
+    d.cnt = (nX + 8 - wave + GQ_WAVES - 1) / GQ_WAVES;
+    d.slot = 16u * (uint32_t)lane;
+    d.ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+    d.stage = stage; d.nst = nst; d.tile0 = tile0;
+  } else {
     const int nI = nX + 8;
     d.cnt = 0;
 #pragma unroll
@@ -453,30 +516,31 @@ __global__ __launch_bounds__(GQ_WAVES * 64, 2) void k_logits_gqa_kernel(const KA
   }
   const int kv = item_kv(itm);
   const int nk = (H.hrank[slot] + 15) >> 4;
-  if (nk <= 2) gq_consume<XT, OUTK, 2, MASKED>(a, H, d, ring, carry, slot, p, kv, b, chunk, ntl, ahead);
-  else if (nk <= 4) gq_consume<XT, OUTK, 4, MASKED>(a, H, d, ring, carry, slot, p, kv, b, chunk, ntl, ahead);
-  else if (nk <= 6) gq_consume<XT, OUTK, 6, MASKED>(a, H, d, ring, carry, slot, p, kv, b, chunk, ntl, ahead);
-  else gq_consume<XT, OUTK, 8, MASKED>(a, H, d, ring, carry, slot, p, kv, b, chunk, ntl, ahead);
+  if (nk <= 2) gq_consume<XT, OUTK, 2, MASKED, LIN>(a, H, d, ring, carry, slot, p, kv, b, chunk, ntl, ahead);
+  else if (nk <= 4) gq_consume<XT, OUTK, 4, MASKED, LIN>(a, H, d, ring, carry, slot, p, kv, b, chunk, ntl, ahead);
+  else if (nk <= 6) gq_consume<XT, OUTK, 6, MASKED, LIN>(a, H, d, ring, carry, slot, p, kv, b, chunk, ntl, ahead);
+  else gq_consume<XT, OUTK, 8, MASKED, LIN>(a, H, d, ring, carry, slot, p, kv, b, chunk, ntl, ahead);
 }
 
-template <typename XT, int OUTK>
+template <typename XT, int OUTK, bool LIN>
 static void launch_gqa_o(const KArgs& a, dim3 grid, dim3 block, hipStream_t st) {
-  if (a.mask != nullptr) hipLaunchKernelGGL((k_logits_gqa_kernel<XT, OUTK, true>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((k_logits_gqa_kernel<XT, OUTK, false>), grid, block, 0, st, a);
+  if (a.mask != nullptr) hipLaunchKernelGGL((k_logits_gqa_kernel<XT, OUTK, true, LIN>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((k_logits_gqa_kernel<XT, OUTK, false, LIN>), grid, block, 0, st, a);
 }
 
-template <typename XT>
+template <typename XT, bool LIN>
 static int launch_gqa_t(const KArgs& a, int outk, int B, hipStream_t st) {
   dim3 grid(a.n_chunks, a.n_wg, B), block(GQ_WAVES * 64);
-  if (outk == 0) launch_gqa_o<XT, 0>(a, grid, block, st);
-  else if (outk == 1) launch_gqa_o<XT, 1>(a, grid, block, st);
-  else launch_gqa_o<XT, 2>(a, grid, block, st);
+  if (outk == 0) launch_gqa_o<XT, 0, LIN>(a, grid, block, st);
+  else if (outk == 1) launch_gqa_o<XT, 1, LIN>(a, grid, block, st);
+  else launch_gqa_o<XT, 2, LIN>(a, grid, block, st);
   return (int)hipGetLastError();
 }
 
 int launch_k_logits_gqa(const KArgs& a, int dtype, bool out_f32, int out_dtype, int B, hipStream_t st) {
   const int outk = out_f32 ? 0 : (out_dtype == STARKV_F16 ? 1 : 2);
-  return dtype == STARKV_F16 ? launch_gqa_t<_Float16>(a, outk, B, st) : launch_gqa_t<__bf16>(a, outk, B, st);
+  if (a.klin) return dtype == STARKV_F16 ? launch_gqa_t<_Float16, true>(a, outk, B, st) : launch_gqa_t<__bf16, true>(a, outk, B, st);
+  return dtype == STARKV_F16 ? launch_gqa_t<_Float16, false>(a, outk, B, st) : launch_gqa_t<__bf16, false>(a, outk, B, st);
 }
 
 }  // namespace starkv

@@ -12,7 +12,9 @@
 //   workgroup) with global_load_lds: 16 bytes per lane, 1 KB per
 //   instruction, only as many instructions as the workgroup's chunks need.
 //   Rows are stored with their 16-byte chunks rotated (ws_shift) so the
-//   consumers' row-wise reads are free of LDS bank conflicts.
+//   consumers' row-wise reads are free of LDS bank conflicts.  A head whose
+//   contiguous rows are not aligned whole chunks (KArgs::klin) is staged as
+//   the run of bytes it is and read from LDS unaligned.
 // * Consumer waves.  The plan packs whole heads into bins of up to 4 items
 //   (query head, 32-rank M-tile), 4 bins per workgroup.
 //   - Dense latents: 4 consumer waves, one per SIMD, wave c runs bin c.  Its
@@ -203,7 +205,8 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
 #pragma unroll
       for (int k = 0; k < WS_MAXH; ++k)
         if (k == nh) { hkv[k] = kv; hrank[k] = r; hoff[k] = tot; }
-      tot += 32 * ws_n16<XI8>(r);           // 16-byte chunks per 32-row tile
+      // 16-byte chunks per 32-row tile
+      tot += !XI8 && ((a.klin >> kv) & 1) ? lin_chunks(r) : 32 * ws_n16<XI8>(r);
       ++nh;
     }
   }
@@ -262,6 +265,18 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
 #pragma unroll
       for (int j = 1; j < WS_MAXH; ++j)
         if (hoff[j] <= q) { hb = hoff[j]; hr = hrank[j]; hk = hkv[j]; }
+      if (!XI8 && ((a.klin >> hk) & 1)) {
+        // linear tile: its bytes as they lie, in aligned 16-byte pieces
+        const char* head = (const char*)a.x + (b * a.x_sb + a.xoff[hk]) * 2;
+        const int mis = (int)((uintptr_t)head & 15);
+        src[k] = head - mis;
+        adv[k] = 16;
+        rowpos[k] = min(q - hb, (mis + 64 * hr - 1) >> 4);
+        tmul[k] = 4 * hr;
+        pmax[k] = (int)((mis + (int64_t)2 * hr * S - 1) >> 4);
+        dst[k] = m * 1024;
+        continue;
+      }
       const int n16 = ws_n16<XI8>(hr), loc = q - hb;
       const int row = loc / n16, cr = loc % n16;             // stored (rotated) chunk cr of row
       const int c = (cr - ws_shift(row, n16) % n16 + n16) % n16;   // the row's chunk that lives there
@@ -338,10 +353,12 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
   half8 wr[MAXI][8];
 #pragma unroll
   for (int i = 0; i < MAXI; ++i) {
-    const bool ok = item_valid(it[i]) && jrow < item_nv(it[i]);
     const int qh = item_qh(it[i]), kv = item_kv(it[i]), mt = item_mt(it[i]);
+    const bool lin = !XI8 && ((a.klin >> kv) & 1);
+    const int rank = lin ? lin_rank(a.krank[kv], mt * 4 + (jrow >> 3), jrow & 7) : jrow < item_nv(it[i]) ? mt * 32 + jrow : -1;
+    const bool ok = item_valid(it[i]) && rank >= 0;
     const XT* qrow = (const XT*)a.q + b * a.q_sb + qh * a.q_sh;
-    const XT* brow = (const XT*)a.bk + a.bkoff[kv] + (int64_t)(mt * 32 + jrow) * a.bk_rs;
+    const XT* brow = (const XT*)a.bk + a.bkoff[kv] + (int64_t)max(rank, 0) * a.bk_rs;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       half8 w = half8{};
@@ -389,6 +406,12 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
       const int c1 = nvh > 8 ? c0 + 1 : c0;
       xo0[i] = rowb + ((c0 + sh) % n16) * 16;
       xo1[i] = rowb + ((c1 + sh) % n16) * 16;
+      if ((a.klin >> kv) & 1) {
+        const char* head = (const char*)a.x + (b * a.x_sb + a.xoff[kv]) * 2;
+        const int row0 = hb * 16 + (int)((uintptr_t)head & 15) + t * 2 * hr;
+        xo0[i] = row0 + 2 * lin_start(hr, c0);
+        xo1[i] = row0 + 2 * lin_start(hr, c1);
+      }
     }
   }
   float mx[MAXI];
@@ -429,8 +452,8 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
     uint4 x0[MAXI], x1[MAXI];
 #pragma unroll
     for (int j = 0; j < MAXI; ++j) {
-      x0[j] = *(const uint4*)(st + xo0[j]);
-      x1[j] = *(const uint4*)(st + xo1[j]);
+      __builtin_memcpy(&x0[j], st + xo0[j], 16);   // (linear heads: any 2-byte alignment)
+      __builtin_memcpy(&x1[j], st + xo1[j], 16);
     }
     half8 T[8];
 #pragma unroll

@@ -1,0 +1,73 @@
+"""Dense K latents whose rows are contiguous but not 16-byte aligned whole
+chunks (odd ranks, odd offsets, odd context lengths), staged as runs of bytes,
+against the oracle; rows that are not contiguous keep the other routes."""
+import pytest
+import torch
+
+from _util import check_logits, check_output, make_case, oracle_decode, oracle_logits
+
+pytestmark = pytest.mark.gpu
+
+F16, BF16 = torch.float16, torch.bfloat16
+# MHA (one odd rank misaligns every later head, whole-chunk ranks included) and grouped queries (ranks at both ends of the
+# linear range, K-steps of 16 ranks at every remainder); one to many tiles per workgroup, contexts ending inside a tile
+CASES = [
+    ("mha_odd", 3, 8, 8, 1003, [9, 16, 101, 32, 128, 33, 96, 127], 200, F16),
+    ("mha_even", 2, 4, 4, 33, [102, 10, 66, 8], 64, F16),
+    ("mha_bf16", 1, 6, 6, 4099, [15, 17, 31, 64, 65, 88], 40, BF16),
+    ("mha_one_position", 2, 3, 3, 1, [11, 24, 55], 64, F16),
+    ("gqa_odd", 2, 16, 4, 1003, [9, 8, 127, 49], 200, F16),
+    ("gqa_102", 1, 32, 8, 2100, [102] * 8, 64, F16),
+    ("gqa_bf16", 3, 8, 4, 777, [113, 97, 33, 15], 64, BF16),
+    ("gqa_odd_heads", 1, 6, 3, 65, [81, 23, 119], 64, F16),
+    ("gqa_too_wide", 1, 4, 2, 500, [128, 31], 64, F16),       # 128 misaligned: copied (K logits) / register streaming
+    ("below_a_chunk", 2, 4, 4, 130, [7, 12, 40, 1], 64, F16),
+]
+
+
+@pytest.mark.parametrize("name,B,Hq,Hkv,S,ranks,Rv,dtype", CASES, ids=[c[0] for c in CASES])
+def test_odd_ranks(name, B, Hq, Hkv, S, ranks, Rv, dtype):
+    from starkv import decode_attention, k_logits
+    print(f"[unaligned rows] {name}", flush=True)
+    case = make_case(B, Hq, Hkv, S, ranks, Rv, dtype=dtype, seed=11)
+    scale = 128 ** -0.5
+    check_logits(k_logits(case.q, case.kspec, S, scale=scale), oracle_logits(case, scale=scale), scale, name)
+    out = decode_attention(case.q, case.kspec, case.xv, case.uv, out_dtype=torch.float32)
+    check_output(out, oracle_decode(case)[0], name)
+
+
+@pytest.mark.parametrize("Hq,Hkv,ranks", [(4, 4, [40, 24, 128, 64]), (8, 2, [104, 56]), (4, 4, [41, 15, 99, 12]),
+                                          (8, 2, [101, 57])])
+@pytest.mark.parametrize("shift", [1, 3, 7])
+def test_shifted_base(Hq, Hkv, ranks, shift):
+    """Rows from a base 2, 6 or 14 bytes off, with infinities planted just
+    outside every head's rows: nothing of them may reach a logit."""
+    from starkv import KLatentSpec, k_logits
+    S, B = 100, 2
+    case = make_case(B, Hq, Hkv, S, ranks, 64, dtype=F16, seed=12)
+    gap = 5
+    sizes = [S * r for r in ranks]
+    buf = torch.full((B, shift + sum(sizes) + gap * Hkv + 8), float("inf"), dtype=F16, device="cuda")
+    offs, o = [], shift
+    for h, n in enumerate(sizes):
+        offs.append(o)
+        buf[:, o:o + n] = case.xk_heads[h].reshape(B, n)
+        o += n + gap
+    k = KLatentSpec(buf, ranks, offs, ranks, buf.stride(0), case.kspec.bk, case.kspec.bk_head_offset,
+                    case.kspec.bk_row_stride)
+    print(f"[shifted base] {shift} {ranks}", flush=True)
+    a, b = k_logits(case.q, k, S), k_logits(case.q, case.kspec, S)
+    # the same products in the same order, whatever the alignment
+    assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("layout_ranks", [[33, 48, 7, 101], [30, 42, 50, 66]])
+def test_rows_not_contiguous(layout_ranks):
+    """All heads of a position side by side (odd ranks): not a linear run."""
+    from starkv import decode_attention, k_logits
+    case = make_case(2, 8, 4, 333, layout_ranks, 64, dtype=F16, layout="posmajor", seed=13)
+    print(f"[posmajor] {layout_ranks}", flush=True)
+    scale = 128 ** -0.5
+    check_logits(k_logits(case.q, case.kspec, 333, scale=scale), oracle_logits(case, scale=scale), scale, "posmajor")
+    check_output(decode_attention(case.q, case.kspec, case.xv, case.uv, out_dtype=torch.float32), oracle_decode(case)[0],
+                 "posmajor")
