@@ -55,6 +55,15 @@ __device__ inline uint4 ld_stream16(const void* p) {
   return make_uint4(t.x, t.y, t.z, t.w);
 }
 
+// eight 16-bit values moved down by n (0..7) places
+__device__ inline uint4 shr_elems(uint4 u, int n) {
+  const uint64_t lo = (uint64_t)u.x | ((uint64_t)u.y << 32), hi = (uint64_t)u.z | ((uint64_t)u.w << 32);
+  const int b = 16 * n;
+  const uint64_t l = n == 0 ? lo : n < 4 ? (lo >> b) | (hi << (64 - b)) : hi >> (b - 64);
+  const uint64_t h = n < 4 ? hi >> b : 0;
+  return make_uint4((uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32));
+}
+
 template <int NTW, int VQ>
 struct PVStage {
   uint4 r[VQ == VQ_DENSE ? NTW : 1];   // dense: X_v chunks (16 B = 8 ranks) of this wave's slab
@@ -164,12 +173,15 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
   constexpr int PITCH = NTW * 32 + 8;            // elements per staged row (16-byte pad)
   constexpr int STAGE = 16 * PITCH;              // elements per staged K-step
   constexpr int CPR = NTW * 4;                   // 16-byte chunks per staged row
-  // dense aligned rows are fetched cooperatively: the workgroup's 256 lanes
+  // dense rows are fetched cooperatively: the workgroup's 256 lanes
   // read each K-step's rows as contiguous 16-byte chunks (every 128-byte line
-  // by one instruction) and write them into the owning wave's slab, one
-  // barrier per K-step.  Per-wave column slabs would split lines between waves
+  // by one instruction; rows of any 2-byte alignment, the last chunk of a
+  // rank that is not a multiple of 8 read as the row's last 8 elements and
+  // moved down: element loads of such rows had left the decode call of B3 S5003
+  // Rv 1637 at 111 us against 85) and write them into the owning wave's slab,
+  // one barrier per K-step.  Per-wave column slabs would split lines between waves
   // and, with non-temporal loads, fetch the split lines twice.
-  constexpr bool COOP = VQ == VQ_DENSE && FAST;
+  constexpr bool COOP = VQ == VQ_DENSE;
   __shared__ __attribute__((aligned(16))) uint16_t stage[4][2][STAGE];
   __shared__ float Ms[32];
   __shared__ float Ps[4][32];
@@ -212,10 +224,14 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
   // ---- per-lane staging map: chunk c -> (row, 16-byte column chunk) of the
   // 16 x NTW*32 slab (cooperative: of the workgroup's 16 x 4*NTW*32 block;
   // soff then counts from stage[0][buf] and includes the owning wave)
-  int goff[NTW], soff[NTW], grow[NTW], gcol[NTW];
+  int soff[NTW], grow[NTW], gcol[NTW];
   bool cok[NTW];
   const int cb0 = cb * 4 * CPR;                                  // first chunk column of the workgroup
-  const int ncol = max(1, min(4 * CPR, a.Rv / 8 - cb0));         // chunk columns it covers (cooperative)
+  const int ncol = max(1, min(4 * CPR, (a.Rv + 7) / 8 - cb0));   // chunk columns it covers (cooperative)
+  // unaligned dense rows: places the last chunk of a row moves down by, and
+  // this lane's chunks (bits) that are one
+  const int drop = VQ == VQ_DENSE && !FAST && a.Rv >= 8 ? (8 - (a.Rv & 7)) & 7 : 0;
+  int tail = 0;
 #pragma unroll
   for (int c = 0; c < NTW; ++c) {
     if constexpr (COOP) {
@@ -223,15 +239,14 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
       const int row = f / ncol, cc = f % ncol;
       grow[c] = row;
       gcol[c] = (cb0 + cc) * 8;
-      goff[c] = 0;
       soff[c] = (cc / CPR) * 2 * STAGE + row * PITCH + (cc % CPR) * 8;
       cok[c] = true;
+      if (gcol[c] + 8 > a.Rv) tail |= 1 << c;
     } else {
       const int f = c * 64 + lane;
       const int row = f / CPR, c16 = f % CPR;
       grow[c] = row;
       gcol[c] = col0 + c16 * 8;
-      goff[c] = row * (int)a.x_ss + gcol[c];
       soff[c] = row * PITCH + c16 * 8;
       cok[c] = (c16 / 4 < nvt) && (gcol[c] < a.Rv);
     }
@@ -245,7 +260,6 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
       if (wave * CPR + c16 >= ncol) *(uint4*)&stage[wave][bf][row * PITCH + c16 * 8] = make_uint4(0, 0, 0, 0);
     }
   }
-  const VT* xb = (const VT*)a.x + b * a.x_sb + (int64_t)s_begin * a.x_ss;
   // quantised: byte offset of the chunk in its row, its block, int8 or int4, its group
   int qoff[NTW], qg[NTW];
   bool qlo[NTW], q8[NTW];
@@ -268,10 +282,17 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
   const char* xrow0 = (const char*)a.x + (b * a.x_sb + (int64_t)s_begin * a.x_ss) * (VQ == VQ_DENSE ? (int64_t)sizeof(VT) : 1);
   const char* srow0 = (const char*)a.xs + (b * a.xs_sb + (int64_t)s_begin * a.xs_ss) * 2;
   const char* zrow0 = (const char*)a.xz + (b * a.xs_sb + (int64_t)s_begin * a.xs_ss) * 2;
+  // chunks of which some lane of this wave holds a row's last (uniform)
+  const uint64_t tails = __builtin_amdgcn_ballot_w64(tail != 0);
+  int wtail = 0;
+  if (VQ == VQ_DENSE && !FAST && tails != 0 && drop != 0) {
+#pragma unroll
+    for (int c = 0; c < NTW; ++c) wtail |= (__builtin_amdgcn_ballot_w64((tail >> c) & 1) != 0) << c;
+  }
   uint32_t xco[NTW], sco[NTW];
 #pragma unroll
   for (int c = 0; c < NTW; ++c) {
-    xco[c] = !cok[c] ? 0u : VQ == VQ_DENSE ? (uint32_t)(gcol[c] * sizeof(VT)) : (uint32_t)qoff[c];
+    xco[c] = !cok[c] ? 0u : VQ == VQ_DENSE ? (uint32_t)((gcol[c] - ((tail >> c) & 1 ? drop : 0)) * sizeof(VT)) : (uint32_t)qoff[c];
     sco[c] = cok[c] ? (uint32_t)qg[c] * 2 : 0u;
   }
 
@@ -324,19 +345,18 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
 #pragma unroll
     for (int c = 0; c < NTW; ++c) {
       if constexpr (VQ != VQ_DENSE) break;
+      const uint32_t ru = (uint32_t)min(kc * KSTEP + grow[c], rmax);
       if (FAST) {
-        const uint32_t ru = (uint32_t)min(kc * KSTEP + grow[c], rmax);
         st.r[c] = ld_stream16(xrow0 + (__umul24(ru, xp) + xco[c]));
+      } else if (a.Rv >= 8) {
+        // (a chunk of rows stays below 2 GB, whatever the pitch)
+        __builtin_memcpy(&st.r[c], xrow0 + (ru * xp + xco[c]), 16);
       } else {
-        const int s0 = s_begin + ks * KSTEP;
-        st.r[c] = make_uint4(0, 0, 0, 0);
-        if (cok[c] && s0 + grow[c] < s_end) {
-          const VT* p = xb + (int64_t)ks * KSTEP * a.x_ss + goff[c];
-          uint16_t tmp[8];
+        const uint16_t* row = (const uint16_t*)(xrow0 + ru * xp);
+        uint32_t w[8];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) tmp[e] = (gcol[c] + e < a.Rv) ? ((const uint16_t*)p)[e] : (uint16_t)0;
-          st.r[c] = make_uint4(tmp[0] | (tmp[1] << 16), tmp[2] | (tmp[3] << 16), tmp[4] | (tmp[5] << 16), tmp[6] | (tmp[7] << 16));
-        }
+        for (int e = 0; e < 8; ++e) w[e] = row[min(e, a.Rv - 1)];
+        st.r[c] = make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16));
       }
     }
     if constexpr (FUSED) {
@@ -373,9 +393,12 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
 #pragma unroll
     for (int c = 0; c < NTW; ++c) {
       if constexpr (COOP) {
-        *(uint4*)&stage[0][buf][soff[c]] = st.r[c];
-      } else if constexpr (VQ == VQ_DENSE) {
-        *(uint4*)&sbuf[soff[c]] = st.r[c];
+        uint4 v = st.r[c];
+        if (!FAST && ((wtail >> c) & 1)) {
+          const uint4 d = shr_elems(v, drop);
+          if ((tail >> c) & 1) v = d;
+        }
+        *(uint4*)&stage[0][buf][soff[c]] = v;
       } else {
         uint4 h = dequant8<VQ>(st.q[c], q8[c], (uint32_t)st.s[c] * 0x10001u,
                                VQ == VQ_G64 ? (uint32_t)st.z[VQ == VQ_G64 ? c : 0] * 0x10001u : 0u);

@@ -71,3 +71,24 @@ def test_rows_not_contiguous(layout_ranks):
     check_logits(k_logits(case.q, case.kspec, 333, scale=scale), oracle_logits(case, scale=scale), scale, "posmajor")
     check_output(decode_attention(case.q, case.kspec, case.xv, case.uv, out_dtype=torch.float32), oracle_decode(case)[0],
                  "posmajor")
+
+
+# V ranks around a chunk, a wave's slab (4, 8 and 13 tiles) and a column block; rows 2-byte aligned
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("Rv,B,S,pad", [(5, 2, 70, 0), (9, 1, 33, 0), (127, 2, 300, 0), (129, 3, 17, 2), (257, 1, 1000, 1),
+                                        (1023, 2, 250, 0), (417, 1, 129, 0), (1249, 2, 200, 0), (1637, 3, 500, 0),
+                                        (1664, 1, 100, 3), (3001, 1, 260, 0)])
+def test_dense_v_rows(Rv, B, S, pad, dtype):
+    """Dense V latents of odd ranks and pitches, in the drop-in P.V and the
+    fused decode; what lies between the rows and past the last is infinite."""
+    from starkv import decode_attention, pv_latent
+    print(f"[dense v rows] Rv={Rv} B={B} S={S} pad={pad} {dtype}", flush=True)
+    case = make_case(B, 8, 8, S, [16] * 8, Rv, dtype=dtype, seed=14)
+    buf = torch.full((B * S * (Rv + pad) + 64,), float("inf"), dtype=dtype, device="cuda")
+    xv = torch.as_strided(buf, (B, S, Rv), (S * (Rv + pad), Rv + pad, 1), 1)
+    xv.copy_(case.xv)
+    p = torch.softmax(torch.randn(B, 8, S, device="cuda", generator=torch.Generator("cuda").manual_seed(1)), -1).to(dtype)
+    ref = torch.matmul(p.double().cpu(), case.xv.double().cpu())
+    check_output(pv_latent(p, xv), ref, "P.V ")
+    out = decode_attention(case.q, case.kspec, xv, case.uv, out_dtype=torch.float32)
+    check_output(out, oracle_decode(case)[0], "decode ")
