@@ -553,8 +553,10 @@ PVGeom pv_geometry(int B, int S, int Rv, bool fused, int vq, int64_t row_bytes) 
   const bool wide = pv_wide_tiles(g.Rvp, fused, vq) > 0 && row_bytes < V_MAX_PITCH;
   // fused group-64 V of up to 16 tiles: the 4-wave raw-nibble kernel, three per CU
   const bool nib4 = fused && vq == VQ_G64 && g.Rvp <= 512;
-  g.n_cb = wide ? 1 : (int)ceil_div(g.Rvp / 32, 4 * ntw);
-  const int wg_per_cu = wide ? 1 : nib4 ? 3 : pv_wg_per_cu(ntw, vq);
+  // the block formats' raw kernel: all columns, one 8-wave workgroup per CU
+  const bool raw = vq == VQ_RAW;
+  g.n_cb = wide || raw ? 1 : (int)ceil_div(g.Rvp / 32, 4 * ntw);
+  const int wg_per_cu = wide || raw ? 1 : nib4 ? 3 : pv_wg_per_cu(ntw, vq);
   const int n_ks = (int)ceil_div(S, KSTEP);
   // each extra split writes and re-reads one fp32 partial of 32 x Rvp per
   // column block, against the X_v bytes and logits the split streams
@@ -567,7 +569,7 @@ PVGeom pv_geometry(int B, int S, int Rv, bool fused, int vq, int64_t row_bytes) 
   g.c2_len = (int)ceil_div(n_ks, n) * KSTEP;
   // the all-columns and raw-nibble kernels take whole 32-position steps (a
   // chunk still below 2 GB)
-  if (wide || nib4) g.c2_len = (int)std::min<int64_t>(round_up(g.c2_len, 2 * KSTEP), std::max<int64_t>(2 * KSTEP, max_ks * KSTEP / (2 * KSTEP) * (2 * KSTEP)));
+  if (wide || nib4 || raw) g.c2_len = (int)std::min<int64_t>(round_up(g.c2_len, 2 * KSTEP), std::max<int64_t>(2 * KSTEP, max_ks * KSTEP / (2 * KSTEP) * (2 * KSTEP)));
   g.n_c2 = (int)ceil_div(S, g.c2_len);
   g.n_grp = g.n_c2 > PV_RG ? (int)ceil_div(g.n_c2, PV_RG) : 0;
   return g;
@@ -699,6 +701,9 @@ int64_t v_row_bytes(const starkv_vlatent& v) {
   return std::max({v.stride_s, v.scale_stride_s * 2, v.stride2_s, v.scale2_stride_s * 2});
 }
 
+// the P.V kernels' storage kind of a validated latent
+int pv_storage(const PVArgs& pa, int vq, int rank) { return vq == VQ_BLOCK && pv_block_ok(pa, rank) ? VQ_RAW : vq; }
+
 int validate_decode(const starkv_decode_desc* d, int* gs, int* n_wg, int* k1pc, int* vq) {
   if (!d) return STARKV_ERR_NULL;
   if (d->batch < 1 || d->seq_len < 1 || d->seq_len > MAX_S) return STARKV_ERR_SHAPE;
@@ -709,6 +714,7 @@ int validate_decode(const starkv_decode_desc* d, int* gs, int* n_wg, int* k1pc, 
   if (st) return st;
   PVArgs vtmp = {};
   if ((st = validate_v(d->v, vtmp, vq))) return st;
+  *vq = pv_storage(vtmp, *vq, d->v.rank);
   if (!d->q || !d->uv || !d->out || !d->rope_table) return STARKV_ERR_NULL;
   if (d->seq_len > d->rope_max_positions) return STARKV_ERR_SHAPE;
   if (d->uv_row_stride < d->v.rank) return STARKV_ERR_SHAPE;
@@ -983,6 +989,7 @@ size_t starkv_pv_latent_workspace_bytes(const starkv_pv_desc* d) {
   PVArgs tmp = {};
   int vq = 0;
   if (validate_v(d->v, tmp, &vq)) return 0;
+  vq = pv_storage(tmp, vq, d->v.rank);
   const int BQ = d->batch * head_groups(d->n_heads);
   const PVGeom g = pv_geometry(BQ, d->seq_len, d->v.rank, false, vq, v_row_bytes(d->v));
   return a256((size_t)BQ * g.n_c2 * 32 * g.Rvp * 4) + a256((size_t)BQ * g.n_grp * 32 * g.Rvp * 4);
@@ -996,6 +1003,7 @@ int starkv_pv_latent(const starkv_pv_desc* d, void* workspace, size_t workspace_
   int st, vq = 0;
   PVArgs a = {};
   if ((st = validate_v(d->v, a, &vq))) return st;
+  vq = pv_storage(a, vq, d->v.rank);
   if (!d->p || !d->out) return STARKV_ERR_NULL;
   const size_t need = starkv_pv_latent_workspace_bytes(d);
   if (!workspace || workspace_bytes < need) return STARKV_ERR_WORKSPACE;
@@ -1056,6 +1064,7 @@ static int decode_impl(const starkv_decode_desc* d, void* workspace, size_t work
 
   PVArgs pa = {};
   if ((st = validate_v(d->v, pa, &vq))) return st;
+  vq = pv_storage(pa, vq, d->v.rank);
   pa.logits = (const float*)(ws + L.off_logits); pa.l_sb = ka.o_sb; pa.l_st = ka.o_st; pa.l_sh = ka.o_sh;
   pa.chunkmax = (const float*)(ws + L.off_cmax); pa.n_chunk1 = L.n_c1;
   pa.part = (float*)(ws + L.off_part); pa.psum = (float*)(ws + L.off_psum); pa.part16 = L.part16;

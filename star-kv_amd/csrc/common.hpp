@@ -102,6 +102,7 @@ constexpr int K1_GQ_RING_BYTES = 81920 - K1_GQ_CARRY_BYTES;    // its LDS ring (
 constexpr int VQ_DENSE = 0;    // act-dtype rows; x strides in elements
 constexpr int VQ_BLOCK = 1;    // per-token fp16 scale: ranks [0, split) in x (int4 nibbles, or int8 when
                                // a_int8), ranks [split, Rv) in x2 (int4 nibbles); x strides in bytes
+constexpr int VQ_RAW = 3;      // VQ_BLOCK storage that pv_block_kernel takes (pv_block_ok)
 constexpr int VQ_G64 = 2;      // int4 asymmetric: fp16 scale and zero per (b, s, 64-rank group)
 
 struct PVArgs {
@@ -427,6 +428,7 @@ int launch_k_logits_ws(const KArgs& a, int dtype, bool out_f32, int out_dtype, i
 int launch_k_logits_gqa(const KArgs& a, int dtype, bool out_f32, int out_dtype, int B, hipStream_t st);
 int launch_pv(const PVArgs& a, int dtype, int vq, bool fused, bool fast, int B, hipStream_t st);
 int pv_tiles_per_wave(int Rvp, bool fused, int vq);   // column tiles (of 32 ranks) per P.V wave
+bool pv_block_ok(const PVArgs& a, int Rv);           // the storage fields (validate_v) are set
 int pv_wide_tiles(int Rvp, bool fused, int vq);       // > 0: the 8-wave all-columns kernel, tiles per wave
 // P.V workgroups resident per CU (the kernel's register budget): the wide
 // dense variants (8 and 13 tiles) take one, the others two

@@ -893,6 +893,12 @@ __device__ inline uint2 lds_read_tr4(const uint8_t* p) {
   return make_uint2((uint32_t)r.x, (uint32_t)r.y);
 }
 
+__device__ inline uint2 lds_read_tr8(const uint8_t* p) {
+  typedef int v2i __attribute__((ext_vector_type(2)));
+  const v2i r = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(p));
+  return make_uint2((uint32_t)r.x, (uint32_t)r.y);
+}
+
 // the LDS row pitch of the raw stage for ngp 64-rank groups: whole groups
 // plus 8 bytes, an odd multiple of 8, so the 16 rows of one transposed read
 // fall on distinct banks; with 16-byte copies (D16) whole groups plus 16
@@ -1198,6 +1204,309 @@ __global__ __launch_bounds__(NWV * 64, (PVNGeom<NWV, NGW, D16>::WGS)) void pv_ni
   }
 }
 
+// P.V over all columns for the per-token block formats (reference int4 with an
+// int8 or int4 upper block, or either alone), the packed rows staged raw.
+//
+// Like pv_nib_kernel: a K-step is 32 positions, the packed bytes go to LDS as
+// they are and are dequantised after a transposed read, each K-step's P is
+// formed once by the workgroup and shared through LDS.  What differs:
+// * rows of any byte alignment (the reference bx default leaves 486-byte lower
+//   rows): the workgroup's 512 threads read each row as unaligned 16-byte
+//   pieces, the last one pulled back to end with the row, into registers two
+//   K-steps ahead, and write them into LDS rows padded for the transposed
+//   reads (tile bytes plus 8, an odd multiple of 8; int8: plus 16, an odd
+//   multiple of 16).  Per-lane dword loads of unaligned rows (a chunk of 8
+//   ranks each) had bound the kernel: 61 us of pv_kernel at B16 S4096 R1228
+//   against 39 us for aligned rows of 1232 ranks; 16-byte pieces are a quarter
+//   of the requests.
+// * int8 tiles are read with ds_read_b64_tr_b8: within a 16-lane group lane j
+//   receives byte j % 8 of the 8 bytes addressed by lanes j / 8 + 2i, i = 0..7.
+//   Even lanes address columns 0..7 of a row, odd lanes columns 8..15, so lane
+//   j receives column j of eight rows.
+// * one scale per token and block: fp16((n - 8) s) or fp16(n s), the integers
+//   exact, one rounding, as the other kernels.
+// Wave w owns up to NT of the column tiles (32 ranks); NP pieces per thread
+// and K-step.  FUSED: P = exp(logit - M) (32-position logit tiles); else P is
+// read as given and the partials are summed by pv_reduce_kernel.
+// (NT by Rvp, and the pieces a row of its launch may have: 16 NP)
+constexpr int PVB_MAX_RV = 1792;                 // 8 tiles a wave spill
+constexpr int pvb_tiles(int Rvp) { return Rvp <= 1024 ? 4 : Rvp <= 1280 ? 5 : 7; }
+constexpr int pvb_max_pieces(int nt) { return nt == 5 ? 48 : 64; }
+__host__ __device__ inline int pvb_pitch(int tiles, bool i8) {
+  return i8 ? 32 * tiles + 16 : 16 * tiles + 8;
+}
+// 16-byte pieces of a row of nb bytes
+__host__ __device__ inline int pvb_pieces(int nb) { return (nb + 15) >> 4; }
+
+template <typename VT, int NT, int NP, bool FUSED>
+__global__ __launch_bounds__(512, 1) void pv_block_kernel(const PVArgs a) {
+  constexpr bool BF = __is_same(VT, __bf16);
+  constexpr int NA = BF && FUSED ? 2 : 1;          // A operand pieces (fused bf16: high and low parts)
+  // two stages of 32 rows of each block (at most 16 NP pieces a row, and the
+  // row pads)
+  constexpr int STAGE = 32 * (256 * NP + 64);
+  __shared__ __attribute__((aligned(16))) uint8_t raw[2 * STAGE];
+  __shared__ __attribute__((aligned(16))) uint16_t Ash[2 * NA * 1024];     // as in pv_nib_kernel
+  __shared__ __attribute__((aligned(16))) uint16_t Ssh[2 * 2 * 2 * 16];    // [buf][block][row half][8 m + 2 pair + row]
+  __shared__ float Ms[32];
+  __shared__ float Ps[32];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, hh = lane >> 5;
+  const int c2 = blockIdx.x, bq = blockIdx.y;
+  const int b = bq / a.n_hg, h0 = (bq - b * a.n_hg) * 32;
+  const int H = a.H;
+  const int s_begin = c2 * a.c2_len;
+  const int s_end = min(a.S, s_begin + a.c2_len);
+  const int len = s_end - s_begin;
+  const int nks = (len + PVN_KS - 1) / PVN_KS;
+
+  // ---- the two blocks: U = ranks [0, split) in x (int8 or int4), L = the rest in x2
+  const bool two = a.split < a.Rv, i8 = a.a_int8;
+  const int nt = a.Rvp / 32, tu = two ? a.split / 32 : nt;                 // column tiles, of them in U
+  const int PU = pvb_pitch(tu, i8), PL = pvb_pitch(nt - tu, false);
+  const int offL = 32 * PU;
+  const int pu = pvb_pieces(a.xnb), pl = two ? pvb_pieces(a.x2nb) : 0;
+
+  // ---- this thread's pieces of a K-step: 32 rows of U, then of L
+  const uint8_t* base[NP];
+  uint32_t pitch[NP];
+  int row[NP], dst[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    const int D = min(tid + 512 * j, 32 * (pu + pl) - 1);                  // past the last piece: it again
+    const bool lo = D >= 32 * pu;
+    const int d = lo ? D - 32 * pu : D, pr = lo ? pl : pu, nb = lo ? a.x2nb : a.xnb;
+    row[j] = d / pr;
+    const int o = min(16 * (d - row[j] * pr), nb - 16);
+    pitch[j] = (uint32_t)(lo ? a.x2_ss : a.x_ss);
+    base[j] = (lo ? (const uint8_t*)a.x2 + b * a.x2_sb + (int64_t)s_begin * a.x2_ss
+                  : (const uint8_t*)a.x + b * a.x_sb + (int64_t)s_begin * a.x_ss) + o;
+    dst[j] = (lo ? offL + row[j] * PL : row[j] * PU) + o;
+  }
+  // ---- P: thread (head eh, ej) forms positions 2 ej, 2 ej + 1
+  const int eh = tid >> 4, ej = tid & 15;
+  const bool hok = h0 + eh < H;
+  const float* lrow = a.logits + b * a.l_sb + (int64_t)min(h0 + eh, H - 1) * a.l_sh + 2 * ej;
+  const VT* prow = (const VT*)a.p + b * a.p_sb + (int64_t)min(h0 + eh, H - 1) * a.p_sh;
+  int aslot[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int p = 2 * ej + u, q = p & 15, q8 = q & 7;
+    aslot[u] = (q >> 3) * 512 + (eh + 32 * (p >> 4)) * 8 + (q8 >> 1) + 4 * (q8 & 1);
+  }
+  // ---- scales: threads 0..63 take (block, row)
+  const bool sth = tid < (two ? 64 : 32);
+  const int sblk = (tid >> 5) & 1, srow = tid & 31;
+  const uint16_t* ssrc = sblk && two ? (const uint16_t*)a.xs2 + b * a.xs2_sb + (int64_t)s_begin * a.xs2_ss
+                                     : (const uint16_t*)a.xs + b * a.xs_sb + (int64_t)s_begin * a.xs_ss;
+  const int64_t sss = sblk && two ? a.xs2_ss : a.xs_ss;
+  const int sdst = (sblk * 2 + (srow >> 4)) * 16 + 8 * ((srow >> 3) & 1) + 4 * (srow & 1) + 2 * ((srow >> 2) & 1) + ((srow >> 1) & 1);
+
+  typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+  typedef u4v u4u __attribute__((aligned(1)));
+  struct Regs { u4v x[NP]; float p[2]; uint16_t s; };
+  // (every load from a clamped, in-bounds row: K-steps past the chunk re-read
+  // its last, rows past s_end its last row; those meet P = 0)
+  auto load = [&](Regs& R, int ks) {
+    const int k0 = min(ks, nks - 1) * PVN_KS;
+#pragma unroll
+    for (int j = 0; j < NP; ++j)
+      R.x[j] = *(const u4u*)(base[j] + __umul24((uint32_t)min(k0 + row[j], len - 1), pitch[j]));
+    if constexpr (FUSED) {
+      const float2 l = *(const float2*)(lrow + (int64_t)((s_begin + k0) >> 5) * a.l_st);   // c2_len: whole 32-position tiles
+      R.p[0] = l.x; R.p[1] = l.y;
+    } else {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) R.p[u] = to_f32(prow[min(s_begin + k0 + 2 * ej + u, s_end - 1)]);
+    }
+    R.s = ssrc[min(k0 + srow, len - 1) * sss];
+  };
+
+  float MqL = 0.f, psum = 0.f;
+  auto publish = [&](const Regs& R, int ks) {
+    const int buf = ks & 1;
+    uint8_t* st = raw + buf * STAGE;
+#pragma unroll
+    for (int j = 0; j < NP; ++j) *(u4u*)(st + dst[j]) = R.x[j];
+    uint16_t* ab = &Ash[buf * NA * 1024];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float ex = FUSED ? __builtin_amdgcn_exp2f(fmaf(R.p[u], 1.4426950408889634f, MqL)) : R.p[u];
+      const float pv = (hok && ks * PVN_KS + 2 * ej + u < len) ? ex : 0.f;
+      psum += pv;
+      if constexpr (!BF) {
+        ab[aslot[u]] = __builtin_bit_cast(uint16_t, (_Float16)pv);
+      } else {
+        const __bf16 hi = (__bf16)pv;                                      // drop-in: exact
+        ab[aslot[u]] = __builtin_bit_cast(uint16_t, hi);
+        if constexpr (FUSED) ab[1024 + aslot[u]] = __builtin_bit_cast(uint16_t, (__bf16)(pv - (float)hi));
+      }
+    }
+    if (sth) Ssh[buf * 64 + sdst] = R.s;
+  };
+
+  // ---- this wave's tiles
+  const int tb = nt / 8, tr = nt % 8;
+  const int ntw = tb + (wave < tr ? 1 : 0), t0 = wave * tb + min(wave, tr);
+  floatx16 acc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) acc[j] = floatx16{};
+  // transposed-read addresses of the lane within a stage (tile 0 of a block)
+  const int r4 = 16 * hh + (lane & 15), c4 = 8 * ((lane >> 4) & 1);
+  const int trU = i8 ? (16 * hh + ((lane & 15) >> 1)) * PU + 16 * ((lane >> 4) & 1) + 8 * (lane & 1) : r4 * PU + c4;
+  const int trL = offL + r4 * PL + c4;
+
+  auto compute = [&](int ks) {
+    const int buf = ks & 1;
+    const uint8_t* st = raw + buf * STAGE;
+    uint4 A[2][NA];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int p = 0; p < NA; ++p) A[m][p] = *(const uint4*)&Ash[(buf * NA + p) * 1024 + m * 512 + 8 * lane];
+    const uint4* sp = (const uint4*)&Ssh[buf * 64 + 16 * hh];
+    uint4 S[2][2];                                                         // [block][m]: 4 row pairs
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) S[u][m] = sp[4 * u + m];
+    auto mul = [&](floatx16& c, const uint32_t (&o)[4], int m) {
+      uint4 bv = make_uint4(o[0], o[1], o[2], o[3]);
+      if constexpr (BF) {
+        bv = f16x8_to_bf16x8(bv);
+#pragma unroll
+        for (int p = 0; p < NA; ++p) c = mfma_bf16(__builtin_bit_cast(bf16x8, A[m][p]), __builtin_bit_cast(bf16x8, bv), c);
+      } else {
+        c = mfma_f16(__builtin_bit_cast(half8, A[m][0]), __builtin_bit_cast(half8, bv), c);
+      }
+    };
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti) {
+      if (ti >= ntw) break;                                                // uniform
+      const int T = t0 + ti;
+      const bool up = T < tu;
+      if (up && i8) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const uint2 w = lds_read_tr8(st + trU + 8 * m * PU + 32 * T);
+          const uint32_t x = w.x ^ 0x80808080u, y = w.y ^ 0x80808080u;     // rows 0..3, 4..7 as n + 128
+          const uint32_t pr[4] = {__builtin_amdgcn_perm(0x64646464u, x, 0x04020400u), __builtin_amdgcn_perm(0x64646464u, y, 0x04020400u),
+                                  __builtin_amdgcn_perm(0x64646464u, x, 0x04030401u), __builtin_amdgcn_perm(0x64646464u, y, 0x04030401u)};
+          const h2v b2 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+          const uint32_t sk[4] = {S[0][m].x, S[0][m].y, S[0][m].z, S[0][m].w};
+          uint32_t o[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) o[k] = as_u32((as_h2(pr[k]) + b2) * as_h2(sk[k]));
+          mul(acc[ti], o, m);
+        }
+      } else {
+        const uint2 w = lds_read_tr4(st + (up ? trU + 16 * T : trL + 16 * (T - tu)));
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const uint32_t wm = m ? w.y : w.x;
+          const uint4 Sm = up ? S[0][m] : S[1][m];
+          const uint32_t lo = wm & 0x0F0F0F0Fu, hi = (wm >> 4) & 0x0F0F0F0Fu;
+          const h2v nv[4] = {__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, false),
+                             __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, true),
+                             __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, false),
+                             __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, true)};
+          const h2v b2 = {(_Float16)-8.0f, (_Float16)-8.0f};
+          const uint32_t sk[4] = {Sm.x, Sm.y, Sm.z, Sm.w};
+          uint32_t o[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) o[k] = as_u32((nv[k] + b2) * as_h2(sk[k]));
+          mul(acc[ti], o, m);
+        }
+      }
+    }
+  };
+
+  // ---- pipeline: registers two K-steps ahead (set k & 1), LDS one ahead
+  // (buffer k & 1).  Iteration k: publish k + 1 (its buffer was last read at
+  // k - 1, before the barrier), load k + 3, compute k, barrier.
+  Regs R[2];
+  load(R[0], 0);
+  load(R[1], 1);
+  if constexpr (FUSED) {
+    const int q = tid >> 3, j = tid & 7;
+    if (tid < 256) {
+      float m = -INFINITY;
+      if (h0 + q < H) m = chunk_max_part(a.chunkmax + ((int64_t)b * H + h0 + q) * a.n_chunk1, a.n_chunk1, j);
+      m = fmaxf(m, __shfl_xor(m, 1, 64));
+      m = fmaxf(m, __shfl_xor(m, 2, 64));
+      m = fmaxf(m, __shfl_xor(m, 4, 64));
+      if (j == 0) Ms[q] = h0 + q < H ? m : 0.f;
+    }
+    __syncthreads();
+    MqL = -Ms[eh] * 1.4426950408889634f;
+  }
+  publish(R[0], 0);
+  load(R[0], 2);
+  __syncthreads();
+  for (int ks = 0; ks < nks; ks += 2) {
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const int k = ks + d;
+      if (d > 0 && k >= nks) break;                                        // uniform
+      publish(R[(d + 1) & 1], k + 1);
+      load(R[(d + 1) & 1], k + 3);
+      compute(k);
+      __syncthreads();
+    }
+  }
+
+  // ---- softmax sums, then the chunk's partial sums (as in pv_kernel)
+  if constexpr (FUSED) {
+#pragma unroll
+    for (int d = 1; d < 16; d *= 2) psum += __shfl_xor(psum, d, 64);
+    if (ej == 0) Ps[eh] = psum;
+    __syncthreads();
+    if (tid < 32) a.psum[((int64_t)bq * a.n_c2 + c2) * 32 + tid] = Ps[tid];
+  }
+  const int64_t prow0 = ((int64_t)bq * a.n_c2 + c2) * 32;
+#pragma unroll
+  for (int ti = 0; ti < NT; ++ti) {
+    if (ti >= ntw) break;
+    const int col = 32 * (t0 + ti) + n;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int q = 8 * (v >> 2) + 4 * hh + (v & 3);
+      if (FUSED && a.part16) {
+        const float sq = Ps[q];
+        ((_Float16*)a.part)[(prow0 + q) * a.Rvp + col] = (_Float16)(acc[ti][v] * (sq > 0.f ? 1.0f / sq : 0.f));
+      } else {
+        a.part[(prow0 + q) * a.Rvp + col] = acc[ti][v];
+      }
+    }
+  }
+}
+
+// Whether the block formats' raw kernel takes this latent: whole tiles in the
+// upper block, rows of at least one 16-byte piece and no more than the
+// kernel's registers hold (an int8 latent past 1024 ranks has too many),
+// 24-bit row pitches.  The others keep pv_wide_kernel and pv_kernel.
+bool pv_block_ok(const PVArgs& a, int Rv) {
+  const bool two = a.split < Rv;
+  if (Rv > PVB_MAX_RV || (two && a.split % 32)) return false;
+  if (a.xnb < 16 || (two && a.x2nb < 16)) return false;
+  const int pieces = pvb_pieces(a.xnb) + (two ? pvb_pieces(a.x2nb) : 0);
+  return pieces <= pvb_max_pieces(pvb_tiles((int)round_up(Rv, 32))) && a.x_ss < (1 << 24) && (!two || a.x2_ss < (1 << 24));
+}
+
+template <typename VT, bool FUSED>
+static void launch_pv_block(const PVArgs& a, int BQ, hipStream_t st) {
+  const bool two = a.split < a.Rv;
+  const int pieces = pvb_pieces(a.xnb) + (two ? pvb_pieces(a.x2nb) : 0);
+  const dim3 grid(a.n_c2, BQ), block(512);
+  const int nt = pvb_tiles(a.Rvp);
+  if (nt == 4 && pieces <= 32) hipLaunchKernelGGL((pv_block_kernel<VT, 4, 2, FUSED>), grid, block, 0, st, a);
+  else if (nt == 4) hipLaunchKernelGGL((pv_block_kernel<VT, 4, 4, FUSED>), grid, block, 0, st, a);
+  else if (nt == 5) hipLaunchKernelGGL((pv_block_kernel<VT, 5, 3, FUSED>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((pv_block_kernel<VT, 7, 4, FUSED>), grid, block, 0, st, a);
+}
+
 // Drop-in path (bx): sum of the chunk partials in fixed chunk order into the
 // act-dtype output.  Each thread sums four columns of a 32x32 output tile;
 // the partial loads are issued eight chunks at a time (32 loads in flight per
@@ -1250,7 +1559,7 @@ int pv_wide_tiles(int Rvp, bool fused, int vq) {
   // fused quantised latents past 32 tiles: the all-columns kernel, 8 waves
   // of ceil(tiles / 8) tiles (B16 S32768 int4-g64, 52 tiles: two column
   // blocks of 4 x 8 tiles fetch the logits and scale rows twice)
-  if (!fused || vq == VQ_DENSE || tiles <= 32 || tiles > 64) return 0;
+  if (!fused || vq == VQ_DENSE || vq == VQ_RAW || tiles <= 32 || tiles > 64) return 0;
   return (tiles + 7) / 8;
 }
 
@@ -1326,7 +1635,8 @@ static int launch_pv_t(const PVArgs& a, int vq, bool fast, int B, hipStream_t st
     hipLaunchKernelGGL((pv_nib_kernel<VT, 4, 2, false>), dim3(a.n_c2, BQ), dim3(256), 0, st, a);
     return (int)hipGetLastError();
   }
-  if (ntw == 4) launch_pv_n<VT, FUSED, 4>(a, vq, fast, BQ, st);
+  if (vq == VQ_RAW) launch_pv_block<VT, FUSED>(a, BQ, st);
+  else if (ntw == 4) launch_pv_n<VT, FUSED, 4>(a, vq, fast, BQ, st);
   else if (ntw == 8) launch_pv_n<VT, FUSED, 8>(a, vq, fast, BQ, st);
   else if constexpr (FUSED) launch_pv_n13<VT>(a, fast, BQ, st);
   int e = (int)hipGetLastError();
