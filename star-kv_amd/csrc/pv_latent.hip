@@ -145,25 +145,54 @@ __device__ inline uint4 f16x8_to_bf16x8(uint4 h) {
   return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// the maximum of one head's K1 chunk maxima cm[0, n) over c = j, j+8, ...:
-// eight independent loads in flight per step (a load-then-max loop would wait
-// out one memory latency per chunk: 32 of them at 256 chunks)
+// the maximum of one head's K1 chunk maxima cm[0, n) over c = j, j+8, ...
+// (j < 8): eight independent loads in flight per step, clamped to the last
+// chunk in the last one (a load-then-max loop waits out one memory latency per
+// chunk, ~2 us each: the maxima were just written by other XCDs)
 __device__ inline float chunk_max_part(const float* cm, int n, int j) {
-  float m[8];
-#pragma unroll
-  for (int u = 0; u < 8; ++u) m[u] = -INFINITY;
-  int c = j;
-  for (; c + 56 < n; c += 64) {
+  float m = -INFINITY;
+  for (int c = j; c < n; c += 64) {
     float v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = cm[c + 8 * u];
+    for (int u = 0; u < 8; ++u) v[u] = cm[min(c + 8 * u, n - 1)];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) m[u] = fmaxf(m[u], v[u]);
+    for (int u = 0; u < 8; ++u) m = fmaxf(m, v[u]);
   }
-  for (; c < n; c += 8) m[0] = fmaxf(m[0], cm[c]);
+  return m;
+}
+
+// One 32 x 32 accumulator tile (lane (n, hh) holds column n of rows
+// 8 g + 4 hh + i, g, i < 4), each row times inv[row] (in LDS) and rounded to
+// fp16, to a row-major array of row pitch `pitch` at column col0: the four
+// lanes of a quad exchange four rows of their four columns, so that lane n
+// stores columns n & ~3 .. + 3 of row 8 g + 4 hh + n % 4 with one instruction.
+// A store takes the address unit a cycle per four lanes whatever its width:
+// 112 2-byte stores per wave spent 6 us of a 29 us launch (B4 S4099 Rv 1640,
+// 128-position chunks; 23 us with these).  fp32 partials gain nothing from it
+// (their dwords already fill the data path; measured 1 us slower).
+template <int SEL> __device__ inline uint32_t quad_xor(uint32_t v) {
+  static_assert(SEL == 1 || SEL == 2, "a lane of the quad");
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, SEL == 1 ? 0xB1 : 0x4E, 0xF, 0xF, true);
+}
+__device__ inline void store_tile_f16(_Float16* out, int64_t pitch, int col0, const floatx16& acc, const float* inv, int lane) {
+  const int n = lane & 31, hh = lane >> 5;
+  const bool b1 = n & 2;
+  // even lanes keep the low halves (row i) of themselves and of lane n ^ 1, odd lanes the high ones (row i + 1)
+  const uint32_t sel = (n & 1) ? 0x07060302u : 0x01000504u;
 #pragma unroll
-  for (int u = 1; u < 8; ++u) m[0] = fmaxf(m[0], m[u]);
-  return m[0];
+  for (int g = 0; g < 4; ++g) {
+    uint32_t p[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int v = 4 * g + 2 * i, q = 8 * g + 4 * hh + 2 * i;
+      const h2v h = {(_Float16)(acc[v] * inv[q]), (_Float16)(acc[v + 1] * inv[q + 1])};
+      const uint32_t own = as_u32(h), other = quad_xor<1>(own);
+      p[i] = __builtin_amdgcn_perm(own, other, sel);
+    }
+    const uint32_t got = quad_xor<2>(b1 ? p[0] : p[1]);
+    const uint2 w = b1 ? make_uint2(got, p[1]) : make_uint2(p[0], got);
+    *(uint2*)(out + (int64_t)(8 * g + 4 * hh + (n & 3)) * pitch + col0 + (n & ~3)) = w;
+  }
 }
 
 template <typename VT, int NTW, bool FUSED, bool FAST, int VQ>
@@ -940,7 +969,7 @@ __global__ __launch_bounds__(NWV * 64, (PVNGeom<NWV, NGW, D16>::WGS)) void pv_ni
   // two rows of pair k of MFMA m (rows 16 hh + 8 m + {0,2}, {4,6}, {1,3}, {5,7})
   __shared__ __attribute__((aligned(16))) uint16_t Ssh[2 * GMAX * 2 * 32];
   __shared__ float Ms[32];
-  __shared__ float Ps[32];
+  __shared__ float Ps[32], Inv[32];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -948,17 +977,6 @@ __global__ __launch_bounds__(NWV * 64, (PVNGeom<NWV, NGW, D16>::WGS)) void pv_ni
   const int c2 = blockIdx.x, bq = blockIdx.y;
   const int b = bq / a.n_hg, h0 = (bq - b * a.n_hg) * 32;
   const int H = a.H;
-
-  if (tid < 256) {
-    const int q = tid >> 3, j = tid & 7;
-    float m = -INFINITY;
-    if (h0 + q < H) m = chunk_max_part(a.chunkmax + ((int64_t)b * H + h0 + q) * a.n_chunk1, a.n_chunk1, j);
-    m = fmaxf(m, __shfl_xor(m, 1, 64));
-    m = fmaxf(m, __shfl_xor(m, 2, 64));
-    m = fmaxf(m, __shfl_xor(m, 4, 64));
-    if (j == 0) Ms[q] = h0 + q < H ? m : 0.f;
-  }
-  __syncthreads();
 
   const int s_begin = c2 * a.c2_len;
   const int s_end = min(a.S, s_begin + a.c2_len);
@@ -1014,7 +1032,7 @@ __global__ __launch_bounds__(NWV * 64, (PVNGeom<NWV, NGW, D16>::WGS)) void pv_ni
   // ---- logits: thread (head eh, ej) takes positions PPT ej .. PPT ej + PPT - 1
   const int eh = tid / TPH, ej = tid % TPH;
   const bool hok = h0 + eh < H;
-  const float MqL = -Ms[eh] * 1.4426950408889634f;
+  float MqL = 0.f;                               // -M log2(e) of the thread's head
   // uniform bases with 32-bit lane offsets (the loads take the scalar-base form)
   const char* lbase = (const char*)(a.logits + b * a.l_sb + (int64_t)h0 * a.l_sh);
   const uint32_t loff = 4u * (uint32_t)(min(eh, H - 1 - h0) * (int)a.l_sh + PPT * ej);
@@ -1150,6 +1168,18 @@ __global__ __launch_bounds__(NWV * 64, (PVNGeom<NWV, NGW, D16>::WGS)) void pv_ni
     copy(V2, 2);
     load(R[0], 0);
     load(R[1], 1);
+    // the heads' maxima, their latency under the first copies'
+    if (tid < 256) {
+      const int q = tid >> 3, j = tid & 7;
+      float m = -INFINITY;
+      if (h0 + q < H) m = chunk_max_part(a.chunkmax + ((int64_t)b * H + h0 + q) * a.n_chunk1, a.n_chunk1, j);
+      m = fmaxf(m, __shfl_xor(m, 1, 64));
+      m = fmaxf(m, __shfl_xor(m, 2, 64));
+      m = fmaxf(m, __shfl_xor(m, 4, 64));
+      if (j == 0) Ms[q] = h0 + q < H ? m : 0.f;
+    }
+    __syncthreads();
+    MqL = -Ms[eh] * 1.4426950408889634f;
     __builtin_amdgcn_s_waitcnt(0);               // vmcnt(0) expcnt(0) lgkmcnt(0)
     publish(R[0], 0);
     for (int ks = 0; ks < nks; ks += 4) {
@@ -1173,33 +1203,26 @@ __global__ __launch_bounds__(NWV * 64, (PVNGeom<NWV, NGW, D16>::WGS)) void pv_ni
   // ---- softmax sums per head (the TPH threads of a head are one wave's lanes)
 #pragma unroll
   for (int d = 1; d < TPH; d *= 2) psum += __shfl_xor(psum, d, 64);
-  if (ej == 0) Ps[eh] = psum;
+  if (ej == 0) {
+    Ps[eh] = psum;
+    Inv[eh] = psum > 0.f ? 1.0f / psum : 0.f;
+  }
   __syncthreads();
   if (tid < 32) a.psum[((int64_t)bq * a.n_c2 + c2) * 32 + tid] = Ps[tid];
-  const int Rvp = a.Rvp;
+  const int64_t p0 = ((int64_t)bq * a.n_c2 + c2) * 32 * a.Rvp;
 #pragma unroll
   for (int gi = 0; gi < NGW; ++gi) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int T = 2 * (g0 + gi) + t;
       if (gi >= ngw || T >= ntile) continue;
-      const int col = 32 * T + n;
       if (a.part16) {
-        _Float16* part = (_Float16*)a.part + (((int64_t)bq * a.n_c2 + c2) * 32) * Rvp;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int q = 8 * (v >> 2) + 4 * hh + (v & 3);
-          const float sq = Ps[q];
-          part[(int64_t)q * Rvp + col] = (_Float16)(acc[2 * gi + t][v] * (sq > 0.f ? 1.0f / sq : 0.f));
-        }
-      } else {
-        float* part = a.part + (((int64_t)bq * a.n_c2 + c2) * 32) * Rvp;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int q = 8 * (v >> 2) + 4 * hh + (v & 3);
-          part[(int64_t)q * Rvp + col] = acc[2 * gi + t][v];
-        }
+        store_tile_f16((_Float16*)a.part + p0, a.Rvp, 32 * T, acc[2 * gi + t], Inv, lane);
+        continue;
       }
+      float* part = a.part + p0 + 32 * T + n;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) part[(int64_t)(8 * (v >> 2) + 4 * hh + (v & 3)) * a.Rvp] = acc[2 * gi + t][v];
     }
   }
 }
@@ -1249,7 +1272,7 @@ __global__ __launch_bounds__(512, 1) void pv_block_kernel(const PVArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t Ash[2 * NA * 1024];     // as in pv_nib_kernel
   __shared__ __attribute__((aligned(16))) uint16_t Ssh[2 * 2 * 2 * 16];    // [buf][block][row half][8 m + 2 pair + row]
   __shared__ float Ms[32];
-  __shared__ float Ps[32];
+  __shared__ float Ps[32], Inv[32];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1461,25 +1484,24 @@ __global__ __launch_bounds__(512, 1) void pv_block_kernel(const PVArgs a) {
   if constexpr (FUSED) {
 #pragma unroll
     for (int d = 1; d < 16; d *= 2) psum += __shfl_xor(psum, d, 64);
-    if (ej == 0) Ps[eh] = psum;
+    if (ej == 0) {
+      Ps[eh] = psum;
+      Inv[eh] = psum > 0.f ? 1.0f / psum : 0.f;
+    }
     __syncthreads();
     if (tid < 32) a.psum[((int64_t)bq * a.n_c2 + c2) * 32 + tid] = Ps[tid];
   }
-  const int64_t prow0 = ((int64_t)bq * a.n_c2 + c2) * 32;
+  const int64_t p0 = ((int64_t)bq * a.n_c2 + c2) * 32 * a.Rvp;
 #pragma unroll
   for (int ti = 0; ti < NT; ++ti) {
     if (ti >= ntw) break;
-    const int col = 32 * (t0 + ti) + n;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int q = 8 * (v >> 2) + 4 * hh + (v & 3);
-      if (FUSED && a.part16) {
-        const float sq = Ps[q];
-        ((_Float16*)a.part)[(prow0 + q) * a.Rvp + col] = (_Float16)(acc[ti][v] * (sq > 0.f ? 1.0f / sq : 0.f));
-      } else {
-        a.part[(prow0 + q) * a.Rvp + col] = acc[ti][v];
-      }
+    if (FUSED && a.part16) {
+      store_tile_f16((_Float16*)a.part + p0, a.Rvp, 32 * (t0 + ti), acc[ti], Inv, lane);
+      continue;
     }
+    float* part = a.part + p0 + 32 * (t0 + ti) + n;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) part[(int64_t)(8 * (v >> 2) + 4 * hh + (v & 3)) * a.Rvp] = acc[ti][v];
   }
 }
 
