@@ -738,11 +738,20 @@ __global__ __launch_bounds__(256, 1) void recon_v_kernel(const PFArgs a) {
 
 // ---------------------------------------------------------------------------
 // Causal flash attention over the reconstructed K / V.  Workgroup: 8 waves x
-// 32 queries of one (b, query head); key blocks of 64 staged in LDS, the next
-// block loaded into registers while the current one is computed.  Per block
-// and wave: S^T = K . Q^T as two 32-key MFMA tiles, the online softmax (the
-// causal mask only on blocks that reach past the wave's first query; blocks
-// wholly in the wave's future skipped), then O^T += V^T . P^T.  The running
+// 32 queries of one (b, query head); key blocks of 64 staged in LDS through
+// registers.  Per block and wave: S^T = K . Q^T as two 32-key MFMA tiles, the
+// online softmax (the causal mask only on blocks that reach past the wave's
+// first query; blocks wholly in the wave's future skipped), then O^T += V^T .
+// P^T.  The loop is pipelined over the blocks: the next block's S^T runs on
+// the matrix cores while this block's exponentials run on the VALU, and its
+// maxima under this block's P.V; K is therefore staged one block ahead of V.
+// Bounds: matrix cores 54 %, LDS 60 % and VALU 46 % of the busy time (B2 T777
+// behind 3001 positions), in near balance; on long prompts the power limit
+// (the whole prefill runs at 0.92 PFLOP/s where a large fp16 matrix product
+// reaches 1.16).  Against one block after another: B8 T8192 6032 -> 5909 us a
+// call, the T777 chunk 166 -> 161 us (same box, results bit-identical);
+// scheduling-group patterns, exponentials spread over the P.V too, and V rows
+// at a 160-half pitch measured the same.  The running
 // maximum moves only when a block's maximum exceeds it by more than
 // 2^FA_RESCALE_LOG2 in exp2 units, so the O rescale is rare and every
 // probability stays <= 2^FA_RESCALE_LOG2 (exact in the final O / l).
@@ -808,97 +817,212 @@ __global__ __launch_bounds__(FA_WAVES * 64, 1) void fa_causal_kernel(const PFArg
   // staging: thread piece i (of 2) covers key 32 i + tid / 16, dims (tid % 16) * 8 .. + 7
   static_assert(FA_KB * 16 == 2 * FA_WAVES * 64, "two 16-byte pieces per thread and tensor");
   const int skey = tid >> 4, sd8 = (tid & 15) * 8;
-  const size_t so0 = (size_t)skey * HEAD_DIM + sd8, so1 = so0 + (size_t)32 * HEAD_DIM;
+  const uint32_t sg = (uint32_t)(skey * HEAD_DIM + sd8) * sizeof(KVT);
   const int lo0 = skey * WT_PITCH + sd8, lo1 = lo0 + 32 * WT_PITCH;
   const int vo0 = skey * FA_VPITCH + sd8, vo1 = vo0 + 32 * FA_VPITCH;
-  // K / V pieces in flight (plain variables: they stay in registers)
-  uint4 k0 = *(const uint4*)(kg + so0), k1 = *(const uint4*)(kg + so1);
-  uint4 v0 = *(const uint4*)(vg + so0), v1 = *(const uint4*)(vg + so1);
-  *(uint4*)&Ks[0][lo0] = k0; *(uint4*)&Ks[0][lo1] = k1;
-  *(uint4*)&Vs[0][vo0] = v0; *(uint4*)&Vs[0][vo1] = v1;
+  uint4 p0, p1;                                     // K or V pieces in flight (plain variables: they stay in registers)
+  {
+    auto at = [&](const KVT* base, int blk, int half) {
+      return *(const uint4*)((const char*)(base + (size_t)min(blk, nkb - 1) * FA_KB * HEAD_DIM) + sg + half * 32 * HEAD_DIM * sizeof(KVT));
+    };
+    const uint4 a0 = at(kg, 0, 0), a1 = at(kg, 0, 1), b0 = at(kg, 1, 0), b1 = at(kg, 1, 1);
+    const uint4 c0 = at(vg, 0, 0), c1 = at(vg, 0, 1);
+    *(uint4*)&Ks[0][lo0] = a0; *(uint4*)&Ks[0][lo1] = a1;
+    *(uint4*)&Ks[1][lo0] = b0; *(uint4*)&Ks[1][lo1] = b1;
+    *(uint4*)&Vs[0][vo0] = c0; *(uint4*)&Vs[0][vo1] = c1;
+  }
   // every load so far (Q included) complete: the loop's MFMAs then wait only
   // on LDS, never on the next block's loads in flight
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int buf = kb & 1;
-    const bool more = kb + 1 < nkb;
-    if (more) {
-      const size_t go = (size_t)(kb + 1) * FA_KB * HEAD_DIM;
-      k0 = *(const uint4*)(kg + go + so0); k1 = *(const uint4*)(kg + go + so1);
-      v0 = *(const uint4*)(vg + go + so0); v1 = *(const uint4*)(vg + go + so1);
-    }
-    if (kb * FA_KB <= w_last) {                     // wave-uniform: the block has keys this wave sees
-      // the two key tiles' MFMA chains interleaved, all 16 K fragments read up front
-      floatx16 s[2] = {floatx16{}, floatx16{}};
-      const uint16_t* kbase = &Ks[buf][n * WT_PITCH + 8 * hh];
-      uint4 kf[2][8];
+  const int nkw = w_last / FA_KB + 1;               // key blocks this wave sees (at most nkb)
+
+  // logits of one key block: two 32-key tiles; lane: keys 64 blk + 32 kt +
+  // 8 (v/4) + 4 hh + v%4 of query t
+  auto qk = [&](const uint16_t* Kb, floatx16 (&s)[2]) {
+    const uint16_t* kbase = Kb + n * WT_PITCH + 8 * hh;
+    s[0] = floatx16{};
+    s[1] = floatx16{};
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) kf[kt][k] = *(const uint4*)(kbase + kt * 32 * WT_PITCH + 16 * k);
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) s[kt] = pf_mfma<KVT>(kf[kt][k], Qb[k], s[kt]);
-      // lane: keys kb*64 + 32 kt + 8 (v/4) + 4 hh + v%4 of query t
-      if (kb * FA_KB + FA_KB - 1 > w_first) {         // the block reaches past some query of the wave
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int key = kb * FA_KB + 32 * kt + 8 * (v >> 2) + 4 * hh + (v & 3);
-            if (key > P) s[kt][v] = -INFINITY;
-          }
-      }
-      float mb = -INFINITY;
+    for (int k = 0; k < 8; ++k)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
+        s[kt] = pf_mfma<KVT>(*(const uint4*)(kbase + kt * 32 * WT_PITCH + 16 * k), Qb[k], s[kt]);
+  };
+  auto row_max = [&](const floatx16 (&s)[2]) -> float {
+    float mb = -INFINITY;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) mb = fmaxf(mb, s[kt][v]);
-      mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
-      if (__ballot(mb > m + thr)) {                  // some query of the wave moves its maximum
-        const float mn = fmaxf(m, mb);                // finite: key 0 <= P in block 0
-        const float alpha = __builtin_amdgcn_exp2f((m - mn) * c);
-        l *= alpha;
+    for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) o[j][v] *= alpha;
-        m = mn;
-      }
-      const float mc = m * c;
-      float ps = 0.f;
+      for (int v = 0; v < 16; ++v) mb = fmaxf(mb, s[kt][v]);
+    return mb;
+  };
+  // before block blk's probabilities: its causal mask and the running maximum
+  auto settle = [&](int blk, floatx16 (&s)[2], float mb) {
+    if (blk * FA_KB + FA_KB - 1 > w_first) {         // the block reaches past some query of the wave
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          s[kt][v] = __builtin_amdgcn_exp2f(fmaf(s[kt][v], c, -mc));
-          ps += s[kt][v];
+          const int key = blk * FA_KB + 32 * kt + 8 * (v >> 2) + 4 * hh + (v & 3);
+          if (key > P) s[kt][v] = -INFINITY;
         }
-      l += ps;                                        // this half's keys; halves joined at the end
-      // O^T += V^T . P^T over the block's four 16-key chunks
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const uint16_t* sb = &Vs[buf][(32 * kt + 16 * kk) * FA_VPITCH + tr_off];
-          half8 ph;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) ph[e] = (_Float16)s[kt][8 * kk + e];
-          const uint4 pb = __builtin_bit_cast(uint4, ph);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint2 lo = pf_read_tr16(sb + 32 * j), hi = pf_read_tr16(sb + 32 * j + 8 * FA_VPITCH);
-            o[j] = pf_mfma<KVT>(make_uint4(lo.x, lo.y, hi.x, hi.y), pb, o[j]);
-          }
-        }
+      mb = row_max(s);
     }
-    if (more) {
-      *(uint4*)&Ks[buf ^ 1][lo0] = k0; *(uint4*)&Ks[buf ^ 1][lo1] = k1;
-      *(uint4*)&Vs[buf ^ 1][vo0] = v0; *(uint4*)&Vs[buf ^ 1][vo1] = v1;
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mb), __float_as_uint(mb), false, false);
+    mb = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    if (__ballot(mb > m + thr)) {                    // some query of the wave moves its maximum
+      const float mn = fmaxf(m, mb);                 // finite: key 0 <= P in block 0
+      const float alpha = __builtin_amdgcn_exp2f((m - mn) * c);
+      l *= alpha;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[j][v] *= alpha;
+      m = mn;
     }
-    __syncthreads();                                // next block staged; this one free to overwrite
+  };
+  // 16-key chunk kk of the probabilities, as the P.V MFMA's B operand
+  auto probs = [&](const floatx16 (&s)[2], int kk, float mc, float& ps) -> uint4 {
+    half8 ph;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = __builtin_amdgcn_exp2f(fmaf(s[kk >> 1][8 * (kk & 1) + e], c, -mc));
+      ps += x;
+      ph[e] = (_Float16)x;
+    }
+    return __builtin_bit_cast(uint4, ph);
+  };
+  // operands of 16 dims of both key tiles; of 64 dims of V^T's 16-key chunk kk
+  auto read_k = [&](const uint16_t* Kb, int k, uint4 (&f)[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) f[i] = *(const uint4*)(Kb + n * WT_PITCH + 8 * hh + i * 32 * WT_PITCH + 16 * k);
+  };
+  auto read_v = [&](const uint16_t* Vb, int kk, int jh, uint4 (&f)[2]) {
+    const uint16_t* sb = Vb + 16 * kk * FA_VPITCH + tr_off + 64 * jh;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint2 lo = pf_read_tr16(sb + 32 * j), hi = pf_read_tr16(sb + 32 * j + 8 * FA_VPITCH);
+      f[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    }
+  };
+  // staging in iteration kb: K of block kb + 2, then V of block kb + 1, one
+  // after the other in the same registers (past the last block: the last one
+  // again, into buffers nobody reads any more)
+  auto fetch = [&](const KVT* base, int blk) {
+    const char* g0 = (const char*)(base + (size_t)min(blk, nkb - 1) * FA_KB * HEAD_DIM);
+    asm volatile("" : "+s"(g0));                     // stays a scalar base: the loads take it with the lane's 32-bit offset
+    p0 = *(const uint4*)(g0 + sg);
+    p1 = *(const uint4*)(g0 + sg + 32 * HEAD_DIM * sizeof(KVT));
+  };
+  auto store_k = [&](int buf) { *(uint4*)&Ks[buf][lo0] = p0; *(uint4*)&Ks[buf][lo1] = p1; };
+  auto store_v = [&](int buf) { *(uint4*)&Vs[buf][vo0] = p0; *(uint4*)&Vs[buf][vo1] = p1; };
+  // Block kb (buffers kb & 1 = BUF): s holds its logits, their mask and
+  // maximum settled; K of block kb + 1 and V of block kb are staged.  The next
+  // block's logits nx are formed while this block's probabilities are.
+  auto block = [&](auto bufc, int kb, floatx16 (&s)[2], floatx16 (&nx)[2]) {
+    constexpr int BUF = decltype(bufc)::value;
+    fetch(kg, kb + 2);
+    uint32_t pb[4][4];
+    uint4 f[2][2];
+    const float mc = m * c;
+    float ps = 0.f, mb = -INFINITY;
+    nx[0] = floatx16{};
+    nx[1] = floatx16{};
+    read_k(Ks[BUF ^ 1], 0, f[0]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (k < 7) read_k(Ks[BUF ^ 1], k + 1, f[(k + 1) & 1]);
+      else read_v(Vs[BUF], 0, 0, f[0]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) nx[i] = pf_mfma<KVT>(f[k & 1][i], Qb[k], nx[i]);
+      // four of the block's probabilities (the empty asm keeps their sum and
+      // their conversion here: left alone, the compiler holds them in fp32 to
+      // the end of the block and spills)
+      typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+      half4 ph;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = __builtin_amdgcn_exp2f(fmaf(s[k >> 2][4 * (k & 3) + e], c, -mc));
+        ps += x;
+        ph[e] = (_Float16)x;
+      }
+      const uint2 w = __builtin_bit_cast(uint2, ph);
+      pb[k >> 1][2 * (k & 1)] = w.x;
+      pb[k >> 1][2 * (k & 1) + 1] = w.y;
+      asm volatile("" : "+v"(pb[k >> 1][2 * (k & 1)]), "+v"(pb[k >> 1][2 * (k & 1) + 1]), "+v"(ps));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    store_k(BUF);
+    fetch(vg, kb + 1);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int kk = u >> 1, jh = u & 1;
+      if (u < 7) read_v(Vs[BUF], (u + 1) >> 1, (u + 1) & 1, f[(u + 1) & 1]);
+      const uint4 pk = make_uint4(pb[kk][0], pb[kk][1], pb[kk][2], pb[kk][3]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) o[2 * jh + j] = pf_mfma<KVT>(f[u & 1][j], pk, o[2 * jh + j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mb = fmaxf(mb, nx[u >> 2][4 * (u & 3) + e]);
+      asm volatile("" : "+v"(mb));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    l += ps;                                         // this half's keys; halves joined at the end
+    settle(kb + 1, nx, mb);
+    store_v(BUF ^ 1);
+    __syncthreads();                                 // next blocks staged; these free to overwrite
+  };
+  // the wave's last block
+  auto last = [&](auto bufc, int kb, floatx16 (&s)[2]) {
+    constexpr int BUF = decltype(bufc)::value;
+    fetch(vg, kb + 1);
+    const float mc = m * c;
+    float ps = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const uint4 pk = probs(s, kk, mc, ps);
+#pragma unroll
+      for (int jh = 0; jh < 2; ++jh) {
+        uint4 f[2];
+        read_v(Vs[BUF], kk, jh, f);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) o[2 * jh + j] = pf_mfma<KVT>(f[j], pk, o[2 * jh + j]);
+      }
+    }
+    l += ps;
+    store_v(BUF ^ 1);
+    fetch(kg, kb + 2);
+    store_k(BUF);
+    __syncthreads();
+  };
+  const std::integral_constant<int, 0> i0;
+  const std::integral_constant<int, 1> i1;
+  floatx16 s0[2], s1[2];
+  qk(Ks[0], s0);
+  settle(0, s0, row_max(s0));
+  // (iteration 0 overwrites the K buffer that other waves may still be reading)
+  __syncthreads();
+  int kb = 0;
+  // (one exit: with a second one between the two blocks the compiler keeps O
+  // in two sets of registers and spills)
+  for (; kb + 2 < nkw; kb += 2) {
+    block(i0, kb, s0, s1);
+    block(i1, kb + 1, s1, s0);
+  }
+  if (kb + 1 < nkw) {
+    block(i0, kb, s0, s1);
+    ++kb;
+    last(i1, kb, s1);
+  } else {
+    last(i0, kb, s0);
+  }
+  // blocks wholly in the wave's future: staging only
+  for (++kb; kb < nkb; ++kb) {
+    fetch(kg, kb + 2);
+    store_k(kb & 1);
+    fetch(vg, kb + 1);
+    store_v(~kb & 1);
+    __syncthreads();
   }
   l += __shfl_xor(l, 32, 64);
   if (t < T) {
