@@ -76,9 +76,11 @@ __device__ inline void gq_wait_vm_n(int n) {
 // stages; the kernel orders it with explicit vmcnt waits and barriers.
 // Each statement sets m0 itself (the compiler treats m0 as reserved and
 // ignores it as a clobber; its code for this kernel holds nothing in m0,
-// which tests/test_gqa_m0.py checks on the compiled gfx950 assembly).
+// which tests/test_gqa_m0.py checks on the compiled gfx950 assembly).  A
+// gfx9 LDS DMA needs a wait state after a scalar write of m0, or it may take
+// the value before it; the compiler adds it only to code of its own.
 __device__ inline void gq_dma(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
 }
 
 template <typename XT> struct GqVec;

@@ -1,13 +1,14 @@
 """Build check of the grouped-query K-logit kernel's inline DMA (CPU only).
 
 k_logits_gqa.hip issues its global -> LDS DMA as inline assembly that sets
-m0 (the LDS destination) itself: `s_mov_b32 m0, sN` then
+m0 (the LDS destination) itself: `s_mov_b32 m0, sN`, `s_nop 0` (the wait
+state that an LDS DMA needs after a scalar write of m0), then
 `global_load_lds_dwordx4`.  The compiler treats m0 as reserved and does not
 see the write, so the kernel is correct only while the compiled code keeps
 nothing of its own in m0.  This test compiles the file to gfx950 assembly
 with the library's flags and fails if any instruction other than those
-pairs names m0, if any LDS DMA is not directly preceded by its own m0 write,
-or if an instruction that reads m0 implicitly appears at all.
+triples names m0, if any LDS DMA is not preceded by its own m0 write and wait
+state, or if an instruction that reads m0 implicitly appears at all.
 """
 import os
 import re
@@ -44,12 +45,13 @@ def test_gqa_dma_is_the_only_m0_user(tmp_path):
     for i, ln in enumerate(code):
         names_m0 = re.search(r"\bm0\b", ln) is not None
         if re.match(r"^\s*s_mov_b32\s+m0,\s+s\d+\s*$", ln):
-            assert i + 1 < len(code) and re.match(r"^\s*global_load_lds_dwordx4\s", code[i + 1]), \
-                f"m0 write not followed by the LDS DMA: {ln!r} / {code[i + 1] if i + 1 < len(code) else ''!r}"
+            assert i + 2 < len(code) and re.match(r"^\s*s_nop\s", code[i + 1]) and \
+                re.match(r"^\s*global_load_lds_dwordx4\s", code[i + 2]), \
+                f"m0 write not followed by a wait state and the LDS DMA: {ln!r} / {code[i + 1:i + 3]}"
             pairs += 1
             continue
         assert not names_m0, f"an instruction other than the DMA's own m0 write names m0: {ln!r}"
         if IMPLICIT_M0.match(ln):
-            assert re.match(r"^\s*global_load_lds_dwordx4\s", ln) and i > 0 and \
-                re.match(r"^\s*s_mov_b32\s+m0,", code[i - 1]), f"an m0 reader without its own m0 write: {ln!r}"
+            assert re.match(r"^\s*global_load_lds_dwordx4\s", ln) and i > 1 and \
+                re.match(r"^\s*s_mov_b32\s+m0,", code[i - 2]), f"an m0 reader without its own m0 write: {ln!r}"
     assert pairs > 0, "no inline DMA found: the check no longer sees the kernel it guards"
