@@ -133,7 +133,9 @@ class LlamaCustomAttention(nn.Module):
         elif query_len > 1:
             pos = torch.arange(S, device=q.device)
             kc, ks = self.rope.cos_sin(pos)
-            K = torch.matmul(key_states, k_u.transpose(-2, -1).to(key_states.dtype))
+            # (U_k^T as a contiguous right operand: torch's batched products over a
+            # transposed one have faulted the GPU in bfloat16)
+            K = torch.matmul(key_states, k_u.transpose(-2, -1).contiguous().to(key_states.dtype))
             K = (K * kc.to(K.dtype) + _rotate_half(K) * ks.to(K.dtype)).repeat_interleave(self.num_key_value_groups, 1)
             V = (torch.matmul(value_states, v_u.weight.T).view(*value_states.shape[:-1], self.num_key_value_heads,
                                                                 self.head_dim).transpose(-3, -2))

@@ -120,7 +120,9 @@ class LlamaCustomAttention(nn.Module):
             vx = torch.cat([(vu_q.to(torch.float32) * svu.float()).to(torch.float16),
                             (unpack_uint8_to_int4_signed(vl_q, r4_v).float() * svl.float()).to(torch.float16)], -1)
             kc, ks = self.rope.cos_sin(torch.arange(S, device=q.device))
-            K = torch.matmul(kx.to(dt), k_u.transpose(-2, -1).to(dt))
+            # (U_k^T as a contiguous right operand: torch's batched products over a
+            # transposed one have faulted the GPU in bfloat16)
+            K = torch.matmul(kx.to(dt), k_u.transpose(-2, -1).contiguous().to(dt))
             K = (K * kc.to(dt) + _rotate_half(K) * ks.to(dt)).repeat_interleave(self.num_key_value_groups, 1)
             V = (torch.matmul(vx.to(dt), v_u.weight.T).view(*vx.shape[:-1], self.num_key_value_heads,
                                                             self.head_dim).transpose(-3, -2))
