@@ -74,6 +74,8 @@ struct KArgs {
   // grouped-query variant (k_logits_gqa.hip, 2 <= gs <= 8): K reconstructed
   // once per KV head; item 0 of consumer wave w = item_pack(kv * gs, kv, dim half, 0, 1)
   int gqa, gs;
+  // (16 bits to keep the argument block small; an entry's address is no whole
+  // number of dwords, which scalar loads need: tests/test_scalar_loads.py)
   int16_t krank[K_MAX_KV];
   // dense heads whose tiles are staged as one run of bytes (bit kv; ws_linear
   // in abi.hip): contiguous rows of any rank and alignment

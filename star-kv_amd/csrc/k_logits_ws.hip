@@ -14,7 +14,9 @@
 //   Rows are stored with their 16-byte chunks rotated (ws_shift) so the
 //   consumers' row-wise reads are free of LDS bank conflicts.  A head whose
 //   contiguous rows are not aligned whole chunks (KArgs::klin) is staged as
-//   the run of bytes it is and read from LDS unaligned.
+//   the run of bytes it is and read from LDS unaligned, in an instantiation
+//   of its own (LIN): asking klin per head in the one for aligned rows cost
+//   those ~1 us a launch (B16 S2048, 32 heads of rank 32: 33.3 against 32.4 us).
 // * Consumer waves.  The plan packs whole heads into bins of up to 4 items
 //   (query head, 32-rank M-tile), 4 bins per workgroup.
 //   - Dense latents: 4 consumer waves, one per SIMD, wave c runs bin c.  Its
@@ -162,7 +164,8 @@ __device__ inline void i8_piece(const uint4& w, kh2 s, const floatx16& acc, int 
 //      dequantised bit-exactly to fp16 after the LDS read; the tile's scales
 //      are staged with its rows (one more DMA instruction), so the consumers
 //      issue no global loads
-template <typename XT, int OUTK, bool XI8>
+// LIN: dense latents some of whose heads are staged as runs of bytes (KArgs::klin)
+template <typename XT, int OUTK, bool XI8, bool LIN>
 __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void k_logits_ws_kernel(const KArgs a) {
   constexpr int NCONS = ws_consumers<XI8>();
   constexpr int MAXI = XI8 ? 2 : 4;                  // items per consumer wave
@@ -206,7 +209,7 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
       for (int k = 0; k < WS_MAXH; ++k)
         if (k == nh) { hkv[k] = kv; hrank[k] = r; hoff[k] = tot; }
       // 16-byte chunks per 32-row tile
-      tot += !XI8 && ((a.klin >> kv) & 1) ? lin_chunks(r) : 32 * ws_n16<XI8>(r);
+      tot += LIN && ((a.klin >> kv) & 1) ? lin_chunks(r) : 32 * ws_n16<XI8>(r);
       ++nh;
     }
   }
@@ -265,7 +268,7 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
 #pragma unroll
       for (int j = 1; j < WS_MAXH; ++j)
         if (hoff[j] <= q) { hb = hoff[j]; hr = hrank[j]; hk = hkv[j]; }
-      if (!XI8 && ((a.klin >> hk) & 1)) {
+      if (LIN && ((a.klin >> hk) & 1)) {
         // linear tile: its bytes as they lie, in aligned 16-byte pieces
         const char* head = (const char*)a.x + (b * a.x_sb + a.xoff[hk]) * 2;
         const int mis = (int)((uintptr_t)head & 15);
@@ -353,12 +356,13 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
   half8 wr[MAXI][8];
 #pragma unroll
   for (int i = 0; i < MAXI; ++i) {
+    const bool in_rank = !LIN && item_valid(it[i]) && jrow < item_nv(it[i]);
     const int qh = item_qh(it[i]), kv = item_kv(it[i]), mt = item_mt(it[i]);
-    const bool lin = !XI8 && ((a.klin >> kv) & 1);
+    const bool lin = LIN && ((a.klin >> kv) & 1);
     const int rank = lin ? lin_rank(a.krank[kv], mt * 4 + (jrow >> 3), jrow & 7) : jrow < item_nv(it[i]) ? mt * 32 + jrow : -1;
-    const bool ok = item_valid(it[i]) && rank >= 0;
+    const bool ok = LIN ? item_valid(it[i]) && rank >= 0 : in_rank;
     const XT* qrow = (const XT*)a.q + b * a.q_sb + qh * a.q_sh;
-    const XT* brow = (const XT*)a.bk + a.bkoff[kv] + (int64_t)max(rank, 0) * a.bk_rs;
+    const XT* brow = (const XT*)a.bk + a.bkoff[kv] + (int64_t)(LIN ? max(rank, 0) : mt * 32 + jrow) * a.bk_rs;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       half8 w = half8{};
@@ -406,7 +410,7 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
       const int c1 = nvh > 8 ? c0 + 1 : c0;
       xo0[i] = rowb + ((c0 + sh) % n16) * 16;
       xo1[i] = rowb + ((c1 + sh) % n16) * 16;
-      if ((a.klin >> kv) & 1) {
+      if (LIN && ((a.klin >> kv) & 1)) {
         const char* head = (const char*)a.x + (b * a.x_sb + a.xoff[kv]) * 2;
         const int row0 = hb * 16 + (int)((uintptr_t)head & 15) + t * 2 * hr;
         xo0[i] = row0 + 2 * lin_start(hr, c0);
@@ -452,8 +456,13 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
     uint4 x0[MAXI], x1[MAXI];
 #pragma unroll
     for (int j = 0; j < MAXI; ++j) {
-      __builtin_memcpy(&x0[j], st + xo0[j], 16);   // (linear heads: any 2-byte alignment)
-      __builtin_memcpy(&x1[j], st + xo1[j], 16);
+      if constexpr (LIN) {                   // any 2-byte alignment
+        __builtin_memcpy(&x0[j], st + xo0[j], 16);
+        __builtin_memcpy(&x1[j], st + xo1[j], 16);
+      } else {
+        x0[j] = *(const uint4*)(st + xo0[j]);
+        x1[j] = *(const uint4*)(st + xo1[j]);
+      }
     }
     half8 T[8];
 #pragma unroll
@@ -673,19 +682,24 @@ __global__ __launch_bounds__((ws_consumers<XI8>() + WS_PRODUCERS) * 64, 1) void 
   }
 }
 
-template <typename XT, bool XI8>
+template <typename XT, bool XI8, bool LIN>
 static int launch_ws_t(const KArgs& a, int outk, int B, hipStream_t st) {
   dim3 grid(a.n_chunks, a.n_wg, B), block((ws_consumers<XI8>() + WS_PRODUCERS) * 64);
-  if (outk == 0) hipLaunchKernelGGL((k_logits_ws_kernel<XT, 0, XI8>), grid, block, 0, st, a);
-  else if (outk == 1) hipLaunchKernelGGL((k_logits_ws_kernel<XT, 1, XI8>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((k_logits_ws_kernel<XT, 2, XI8>), grid, block, 0, st, a);
+  if (outk == 0) hipLaunchKernelGGL((k_logits_ws_kernel<XT, 0, XI8, LIN>), grid, block, 0, st, a);
+  else if (outk == 1) hipLaunchKernelGGL((k_logits_ws_kernel<XT, 1, XI8, LIN>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((k_logits_ws_kernel<XT, 2, XI8, LIN>), grid, block, 0, st, a);
   return (int)hipGetLastError();
+}
+
+template <typename XT>
+static int launch_ws_x(const KArgs& a, int outk, int B, hipStream_t st) {
+  if (a.ws_i8) return launch_ws_t<XT, true, false>(a, outk, B, st);
+  return a.klin ? launch_ws_t<XT, false, true>(a, outk, B, st) : launch_ws_t<XT, false, false>(a, outk, B, st);
 }
 
 int launch_k_logits_ws(const KArgs& a, int dtype, bool out_f32, int out_dtype, int B, hipStream_t st) {
   const int outk = out_f32 ? 0 : (out_dtype == STARKV_F16 ? 1 : 2);
-  if (a.ws_i8) return dtype == STARKV_F16 ? launch_ws_t<_Float16, true>(a, outk, B, st) : launch_ws_t<__bf16, true>(a, outk, B, st);
-  return dtype == STARKV_F16 ? launch_ws_t<_Float16, false>(a, outk, B, st) : launch_ws_t<__bf16, false>(a, outk, B, st);
+  return dtype == STARKV_F16 ? launch_ws_x<_Float16>(a, outk, B, st) : launch_ws_x<__bf16>(a, outk, B, st);
 }
 
 }  // namespace starkv
