@@ -209,6 +209,9 @@ int starkv_k_logits(const starkv_klogits_desc* d, void* workspace, size_t worksp
  *     and zero of (b, s, group g = rank/64) at scale / zero + b*scale_stride_b
  *     + s*scale_stride_s + g; x = n*s + z.  Row pitches (stride_s, and
  *     scale_stride_s in bytes) below 16 MB, else STARKV_ERR_LIMIT.
+ * starkv_pv_latent and the decode entry points take dense rows whose first
+ * min(seq_len, 16) positions span less than 2^32 bytes, else
+ * STARKV_ERR_LIMIT (any pitch below 286 MB).
  * ------------------------------------------------------------------- */
 typedef struct {
   int rank;

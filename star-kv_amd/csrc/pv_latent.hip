@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
       if (FAST) {
         st.r[c] = ld_stream16(xrow0 + (__umul24(ru, xp) + xco[c]));
       } else if (a.Rv >= 8) {
-        // (a chunk of rows stays below 2 GB, whatever the pitch)
+        // (a chunk stays below 2 GB, or is one step of less than 4 GB: check_v_step in abi.hip)
         __builtin_memcpy(&st.r[c], xrow0 + (ru * xp + xco[c]), 16);
       } else {
         const uint16_t* row = (const uint16_t*)(xrow0 + ru * xp);

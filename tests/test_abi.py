@@ -265,6 +265,25 @@ def test_rope_build_and_pv_validation():
     assert lib.starkv_pv_latent(ctypes.byref(p), FAKE, need, None) == ERR_LIMIT
 
 
+def test_dense_v_rows_of_a_step_stay_below_4_gb():
+    """P.V addresses the rows of a 16-position step with 32-bit byte offsets:
+    a dense pitch whose step would pass them is refused, not read modulo 2^32."""
+    lib = L.lib()
+    for S, ok, refused in [(16, 143165559, 143165560), (17, 143165559, 143165560), (3, 2 ** 30 - 128, 2 ** 30 - 127),
+                           (2, 2 ** 31 - 256, 2 ** 31 - 255), (1, 2 ** 33, None)]:
+        for pitch, code in ((ok, ERR_WORKSPACE), (refused, ERR_LIMIT)):
+            if pitch is None:
+                continue
+            p = L.PVDesc(batch=1, n_heads=32, seq_len=S, dtype=L.F16, p=FAKE, p_stride_b=3200, p_stride_h=100,
+                         v=L.VLatent(rank=256, format=L.FMT_DENSE, data=FAKE, stride_b=0, stride_s=pitch),
+                         out=FAKE, out_stride_b=8192, out_stride_h=256)
+            assert lib.starkv_pv_latent(ctypes.byref(p), None, 0, None) == code, (S, pitch)
+            assert (lib.starkv_pv_latent_workspace_bytes(ctypes.byref(p)) > 0) == (code == ERR_WORKSPACE)
+            d = _decode_desc([], S=S)
+            d.v.stride_b, d.v.stride_s = 0, pitch
+            assert _call(d) == code, (S, pitch)
+
+
 def test_k_logits_validation():
     lib = L.lib()
     keep = []
