@@ -195,7 +195,9 @@ __device__ inline void store_tile_f16(_Float16* out, int64_t pitch, int col0, co
   }
 }
 
-template <typename VT, int NTW, bool FUSED, bool FAST, int VQ>
+// NC: 16-byte chunks a lane fetches per K-step of unaligned dense rows, for
+// ranks that leave fewer than NTW full ones (pv_lane_chunks)
+template <typename VT, int NTW, bool FUSED, bool FAST, int VQ, int NC = NTW>
 __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PVArgs a) {
   // K-steps of loads in flight per wave (register stages)
   constexpr int DEPTH = VQ == VQ_DENSE ? 2 : PV_QDEPTH;
@@ -253,8 +255,8 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
   // ---- per-lane staging map: chunk c -> (row, 16-byte column chunk) of the
   // 16 x NTW*32 slab (cooperative: of the workgroup's 16 x 4*NTW*32 block;
   // soff then counts from stage[0][buf] and includes the owning wave)
-  int soff[NTW], grow[NTW], gcol[NTW];
-  bool cok[NTW];
+  int soff[NC], grow[NC], gcol[NC];
+  bool cok[NC];
   const int cb0 = cb * 4 * CPR;                                  // first chunk column of the workgroup
   const int ncol = max(1, min(4 * CPR, (a.Rv + 7) / 8 - cb0));   // chunk columns it covers (cooperative)
   // unaligned dense rows: places the last chunk of a row moves down by, and
@@ -262,7 +264,7 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
   const int drop = VQ == VQ_DENSE && !FAST && a.Rv >= 8 ? (8 - (a.Rv & 7)) & 7 : 0;
   int tail = 0;
 #pragma unroll
-  for (int c = 0; c < NTW; ++c) {
+  for (int c = 0; c < NC; ++c) {
     if constexpr (COOP) {
       const int f = min(c * 256 + tid, 16 * ncol - 1);           // lanes past the block repeat its last chunk
       const int row = f / ncol, cc = f % ncol;
@@ -290,14 +292,14 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
     }
   }
   // quantised: byte offset of the chunk in its row, its block, int8 or int4, its group
-  int qoff[NTW], qg[NTW];
-  bool qlo[NTW], q8[NTW];
+  int qoff[NC], qg[NC];
+  bool qlo[NC], q8[NC];
   const uint8_t* xq = (const uint8_t*)a.x + b * a.x_sb + (int64_t)s_begin * a.x_ss;
   const uint8_t* xq2 = (const uint8_t*)a.x2 + b * a.x2_sb + (int64_t)s_begin * a.x2_ss;
   const uint16_t* sq = (const uint16_t*)a.xs + b * a.xs_sb + (int64_t)s_begin * a.xs_ss;
   const uint16_t* sq2 = (const uint16_t*)a.xs2 + b * a.xs2_sb + (int64_t)s_begin * a.xs2_ss;
 #pragma unroll
-  for (int c = 0; c < NTW; ++c) {
+  for (int c = 0; c < NC; ++c) {
     qlo[c] = VQ == VQ_BLOCK && gcol[c] >= a.split;
     q8[c] = VQ == VQ_BLOCK && !qlo[c] && a.a_int8;
     qoff[c] = qlo[c] ? (gcol[c] - a.split) / 2 : (q8[c] ? gcol[c] : gcol[c] / 2);
@@ -316,11 +318,11 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
   int wtail = 0;
   if (VQ == VQ_DENSE && !FAST && tails != 0 && drop != 0) {
 #pragma unroll
-    for (int c = 0; c < NTW; ++c) wtail |= (__builtin_amdgcn_ballot_w64((tail >> c) & 1) != 0) << c;
+    for (int c = 0; c < NC; ++c) wtail |= (__builtin_amdgcn_ballot_w64((tail >> c) & 1) != 0) << c;
   }
-  uint32_t xco[NTW], sco[NTW];
+  uint32_t xco[NC], sco[NC];
 #pragma unroll
-  for (int c = 0; c < NTW; ++c) {
+  for (int c = 0; c < NC; ++c) {
     xco[c] = !cok[c] ? 0u : VQ == VQ_DENSE ? (uint32_t)((gcol[c] - ((tail >> c) & 1 ? drop : 0)) * sizeof(VT)) : (uint32_t)qoff[c];
     sco[c] = cok[c] ? (uint32_t)qg[c] * 2 : 0u;
   }
@@ -332,12 +334,12 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
   // nothing is zeroed, and with a fixed number of loads per stage (no branch
   // in the loop body) the compiler waits for exactly the older stage
   // (vmcnt(n)) instead of draining every load at the loop head.
-  auto load = [&](PVStage<NTW, VQ>& st, int ks) {
+  auto load = [&](PVStage<NC, VQ>& st, int ks) {
     const int kc = min(ks, nks - 1);
     const int rmax = s_end - 1 - s_begin;                   // last valid row of the chunk
     if constexpr (VQ != VQ_DENSE) {
 #pragma unroll
-      for (int c = 0; c < NTW; ++c) {
+      for (int c = 0; c < NC; ++c) {
         const int64_t r = min(kc * KSTEP + grow[c], rmax);
         if constexpr (VQ == VQ_BLOCK) {
           const bool lo = cok[c] && qlo[c];
@@ -372,7 +374,7 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
       }
     }
 #pragma unroll
-    for (int c = 0; c < NTW; ++c) {
+    for (int c = 0; c < NC; ++c) {
       if constexpr (VQ != VQ_DENSE) break;
       const uint32_t ru = (uint32_t)min(kc * KSTEP + grow[c], rmax);
       if (FAST) {
@@ -400,7 +402,8 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
       const int sa = s_begin + ks * KSTEP + 8 * hh;
       const VT* pp = (const VT*)a.p + b * a.p_sb + min(h0 + n, H - 1) * a.p_sh + sa;
       st.praw = make_uint4(0, 0, 0, 0);
-      if (qok && ks < nks) {
+      // (unaligned rows: a wave without columns, of small ranks, only fetches V)
+      if (qok && ks < nks && (FAST || VQ != VQ_DENSE || nvt > 0)) {
         if (a.p_vec && sa + 8 <= s_end) {
           st.praw = *(const uint4*)pp;
         } else {
@@ -417,10 +420,10 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
   const int g = lane >> 4, rho = lane & 15;
   const int tr_off = (8 * hh + (rho >> 2)) * PITCH + 16 * (g & 1) + 4 * (rho & 3);
 
-  auto compute = [&](PVStage<NTW, VQ>& st, int ks, int buf) {
+  auto compute = [&](PVStage<NC, VQ>& st, int ks, int buf) {
     uint16_t* sbuf = &stage[wave][buf][0];
 #pragma unroll
-    for (int c = 0; c < NTW; ++c) {
+    for (int c = 0; c < NC; ++c) {
       if constexpr (COOP) {
         uint4 v = st.r[c];
         if (!FAST && ((wtail >> c) & 1)) {
@@ -509,7 +512,7 @@ __global__ __launch_bounds__(256, pv_wg_per_cu(NTW, VQ)) void pv_kernel(const PV
     // K-steps in groups of DEPTH, each stage loaded DEPTH steps ahead; the
     // last group computes up to DEPTH - 1 K-steps past the chunk with P = 0
     // (no branch in the loop body)
-    PVStage<NTW, VQ> st[DEPTH];
+    PVStage<NC, VQ> st[DEPTH];
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) load(st[d], d);
     for (int ks = 0; ks < nks; ks += DEPTH) {
@@ -1603,6 +1606,13 @@ int pv_tiles_per_wave(int Rvp, bool fused, int vq) {
 // fast: dense rows 16-byte aligned (ranks a multiple of 8); quantised rows
 // aligned for 4-byte (int4) / 8-byte (int8) chunk loads, else the
 // unaligned-row loads
+// Chunks a lane of the unaligned dense kernel fetches per K-step: the 16 rows'
+// chunks over the workgroup's 256 lanes.  With four for every rank up to 512
+// most lanes of a small one fetched, moved and stored its last chunk over and
+// over (P.V of rank 33, B3 S5003: 17.0 us with four, 14.2 with one; rank 127:
+// 18.4 and 15.6; rank 5: 17.8 and 13.3).
+static int pv_lane_chunks(int Rv) { return Rv <= 128 ? 1 : Rv <= 256 ? 2 : 4; }
+
 template <typename VT, bool FUSED, int NTW>
 static void launch_pv_n(const PVArgs& a, int vq, bool fast, int B, hipStream_t st) {
   dim3 grid(a.n_cb * a.n_c2, B), block(256);
@@ -1611,7 +1621,15 @@ static void launch_pv_n(const PVArgs& a, int vq, bool fast, int B, hipStream_t s
   else if (vq == VQ_G64 && fast) hipLaunchKernelGGL((pv_kernel<VT, NTW, FUSED, true, VQ_G64>), grid, block, 0, st, a);
   else if (vq == VQ_G64) hipLaunchKernelGGL((pv_kernel<VT, NTW, FUSED, false, VQ_G64>), grid, block, 0, st, a);
   else if (fast) hipLaunchKernelGGL((pv_kernel<VT, NTW, FUSED, true, VQ_DENSE>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((pv_kernel<VT, NTW, FUSED, false, VQ_DENSE>), grid, block, 0, st, a);
+  else {
+    if constexpr (NTW == 4) {
+      const int nc = pv_lane_chunks(a.Rv);
+      if (nc == 1) hipLaunchKernelGGL((pv_kernel<VT, 4, FUSED, false, VQ_DENSE, 1>), grid, block, 0, st, a);
+      else if (nc == 2) hipLaunchKernelGGL((pv_kernel<VT, 4, FUSED, false, VQ_DENSE, 2>), grid, block, 0, st, a);
+      if (nc < 4) return;
+    }
+    hipLaunchKernelGGL((pv_kernel<VT, NTW, FUSED, false, VQ_DENSE>), grid, block, 0, st, a);
+  }
 }
 
 template <typename VT>

@@ -77,7 +77,9 @@ def test_rows_not_contiguous(layout_ranks):
 @pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("Rv,B,S,pad", [(5, 2, 70, 0), (9, 1, 33, 0), (127, 2, 300, 0), (129, 3, 17, 2), (257, 1, 1000, 1),
                                         (1023, 2, 250, 0), (417, 1, 129, 0), (1249, 2, 200, 0), (1637, 3, 500, 0),
-                                        (1664, 1, 100, 3), (3001, 1, 260, 0)])
+                                        (1664, 1, 100, 3), (3001, 1, 260, 0),
+                                        # one, two and four chunks a lane: their last and first ranks
+                                        (128, 2, 130, 1), (255, 1, 65, 0), (256, 2, 47, 3)])
 def test_dense_v_rows(Rv, B, S, pad, dtype):
     """Dense V latents of odd ranks and pitches, in the drop-in P.V and the
     fused decode; what lies between the rows and past the last is infinite."""
