@@ -174,7 +174,12 @@ bool ws_rows16(const starkv_klatent& k, int h, int xe, bool padded) {
 // 32 heads of odd ranks, B3 S5003: the decode call 148 against 111 us, its K
 // logits 69 us before).  Below 8 ranks a row holds no whole chunk.  The grouped-query kernel stages either
 // all heads of a launch so or none, and its DMA slots hold two linear heads of
-// up to 127 ranks.
+// up to 127 ranks.  decode: up to 8192 positions of one-query heads below 16
+// ranks, fewer than 384 in all, stay with the register-streaming kernel, whose
+// few loads start sooner (decode calls, staged against streamed, us: 32 heads
+// of rank 10, S4099 37.5 / 35.3, S65536 68.6 / 73.3; of rank 14, S4099 37.8 /
+// 38.3; 8 heads of rank 15, S4099 32.4 / 31.7, of rank 20 32.6 / 33.1; 31
+// heads of rank 9 beside one of 127, S4099 36.6 / 42.3).
 bool ws_linear(const starkv_klatent& k, int h, int gs) {
   return k.format == STARKV_FMT_DENSE && k.pos_stride[h] == k.rank[h] && k.rank[h] >= 8 && k.rank[h] <= (gs > 1 ? 127 : 128) &&
          al(k.data, 2);
@@ -185,16 +190,20 @@ struct LinPlan {
   bool ok;
   uint64_t mask;
 };
-LinPlan lin_plan(const starkv_klatent& k, int gs, int xe, bool padded) {
+LinPlan lin_plan(const starkv_klatent& k, int gs, int xe, int S, bool padded, bool decode) {
   LinPlan p = {true, 0};
   bool all = true;
+  int ranks = 0, rmax = 0;
   for (int h = 0; h < k.n_kv_heads; ++h) {
     const bool l = ws_linear(k, h, gs);
     all = all && l;
+    ranks += k.rank[h];
+    rmax = std::max(rmax, k.rank[h]);
     if (ws_rows16(k, h, xe, padded)) continue;
     if (!l) return {false, 0};
     p.mask |= (uint64_t)1 << h;
   }
+  if (p.mask && gs == 1 && decode && rmax < 16 && ranks < 384 && S <= 8192) return {false, 0};
   if (p.mask && gs > 1) {
     if (!all) return {false, 0};
     for (int h = 0; h < k.n_kv_heads; ++h) p.mask |= (uint64_t)1 << h;
@@ -208,7 +217,7 @@ LinPlan lin_plan(const starkv_klatent& k, int gs, int xe, bool padded) {
 // DMA pieces never straddle rows); q and B_k are read element-wise there.
 // padded: dense rows hold round_up(r, 8) elements, zero past r (the K-logit
 // entry's repacked copy), so a rank need not be a multiple of 8.
-bool k_ws(const starkv_klatent& k, int gs, int dtype, int S, bool padded = false) {
+bool k_ws(const starkv_klatent& k, int gs, int dtype, int S, bool padded, bool decode) {
   const bool i8 = k.format == STARKV_FMT_INT8_SYM;
   if (k.format != STARKV_FMT_DENSE && !i8) return false;
   const int xe = i8 ? 1 : esize(dtype);
@@ -223,7 +232,7 @@ bool k_ws(const starkv_klatent& k, int gs, int dtype, int S, bool padded = false
     if (i8 && (k.rank[h] % 8 || !al64(k.head_offset[h], 16) || !al64(k.pos_stride[h], 16))) return false;
     if ((int64_t)TILE * k.pos_stride[h] * xe >= ((int64_t)1 << 31)) return false;   // 32-bit per-tile DMA step
   }
-  return i8 || lin_plan(k, gs, xe, padded).ok;
+  return i8 || lin_plan(k, gs, xe, S, padded, decode).ok;
 }
 
 // 16-byte LDS chunks of one 32-position tile row of a head in that kernel
@@ -344,8 +353,8 @@ static bool ws_balance(const starkv_klatent& k, int Hq, int unit, int nw, int ca
 // and deal the waves round-robin over workgroups of 8 waves (2-item waves) or
 // 4 waves (4-item waves).
 int build_k_plan(const starkv_klatent& k, int Hq, int gs, int dtype, int S, KArgs& a, KPlan& plan,
-                 bool padded = false) {
-  const bool ws = k_ws(k, gs, dtype, S, padded);
+                 bool padded, bool decode) {
+  const bool ws = k_ws(k, gs, dtype, S, padded, decode);
   const int unit = 32;                        // ranks per item
   struct QH { int qh, kv, ni; };              // ni: items of the head
   std::vector<QH> heads;
@@ -468,7 +477,7 @@ int build_k_plan(const starkv_klatent& k, int Hq, int gs, int dtype, int S, KArg
   }
   a.gqa = gqa;
   a.gs = gs;
-  a.klin = ws && k.format == STARKV_FMT_DENSE ? lin_plan(k, gs, esize(dtype), padded).mask : 0;
+  a.klin = ws && k.format == STARKV_FMT_DENSE ? lin_plan(k, gs, esize(dtype), S, padded, decode).mask : 0;
   for (int h = 0; h < K_MAX_KV; ++h) a.krank[h] = (int16_t)(h < k.n_kv_heads ? k.rank[h] : 0);
   const bool two = k.format == STARKV_FMT_INT4_REF && k.split > 0;
   a.ksplit = two ? k.split : 128;
@@ -732,7 +741,7 @@ int validate_decode(const starkv_decode_desc* d, int* gs, int* n_wg, int* k1pc, 
   if (d->out_dtype != 0 && d->out_dtype != d->dtype && d->out_dtype != STARKV_F32) return STARKV_ERR_DTYPE;
   KArgs tmp;
   KPlan plan;
-  if ((st = build_k_plan(d->k, d->n_q_heads, *gs, d->dtype, d->seq_len, tmp, plan))) return st;
+  if ((st = build_k_plan(d->k, d->n_q_heads, *gs, d->dtype, d->seq_len, tmp, plan, false, true))) return st;
   *n_wg = plan.n_wg;
   *k1pc = plan.per_cu;
   return STARKV_OK;
@@ -912,7 +921,7 @@ struct KRepack {
 KRepack k_repack_plan(const starkv_klatent& k, int gs, int dtype, int B, int S) {
   KRepack r;
   if (k.format != STARKV_FMT_DENSE) return r;
-  const bool ws = k_ws(k, gs, dtype, S);
+  const bool ws = k_ws(k, gs, dtype, S, false, false);
   bool rows16 = ws;
   for (int h = 0; h < k.n_kv_heads; ++h) rows16 = rows16 && ws_rows16(k, h, esize(dtype), false);
   if (rows16) return r;
@@ -972,7 +981,7 @@ int starkv_k_logits(const starkv_klogits_desc* d, void* workspace, size_t worksp
   }
   KArgs a;
   KPlan plan;
-  if ((st = build_k_plan(k, d->n_q_heads, gs, d->dtype, d->seq_len, a, plan, rp.on))) return st;
+  if ((st = build_k_plan(k, d->n_q_heads, gs, d->dtype, d->seq_len, a, plan, rp.on, false))) return st;
   a.q = d->q; a.q_sb = d->q_stride_b; a.q_sh = d->q_stride_h;
   a.x = k.data; a.x_sb = k.stride_b;
   a.xscale = d->k.scale; a.xs_sb = d->k.scale_stride_b; a.xs_sh = d->k.scale_stride_h;
@@ -1053,7 +1062,7 @@ static int decode_impl(const starkv_decode_desc* d, void* workspace, size_t work
 
   KArgs ka;
   KPlan plan;
-  if ((st = build_k_plan(d->k, Hq, gs, d->dtype, d->seq_len, ka, plan))) return st;
+  if ((st = build_k_plan(d->k, Hq, gs, d->dtype, d->seq_len, ka, plan, false, true))) return st;
   ka.q = d->q; ka.q_sb = d->q_stride_b; ka.q_sh = d->q_stride_h;
   ka.x = d->k.data; ka.x_sb = d->k.stride_b;
   ka.xscale = d->k.scale; ka.xs_sb = d->k.scale_stride_b; ka.xs_sh = d->k.scale_stride_h;

@@ -22,6 +22,8 @@ CASES = [
     ("gqa_odd_heads", 1, 6, 3, 65, [81, 23, 119], 64, F16),
     ("gqa_too_wide", 1, 4, 2, 500, [128, 31], 64, F16),       # 128 misaligned: copied (K logits) / register streaming
     ("below_a_chunk", 2, 4, 4, 130, [7, 12, 40, 1], 64, F16),
+    ("mha_few_ranks", 2, 6, 6, 300, [8, 9, 13, 15, 11, 14], 64, F16),    # (decode streams them in registers)
+    ("mha_few_ranks_bf16", 1, 5, 5, 129, [10, 11, 12, 14, 15], 40, BF16),
 ]
 
 
