@@ -721,7 +721,9 @@ int check_v_step(const starkv_vlatent& v, int S) {
 }
 
 // the P.V kernels' storage kind of a validated latent
-int pv_storage(const PVArgs& pa, int vq, int rank) { return vq == VQ_BLOCK && pv_block_ok(pa, rank) ? VQ_RAW : vq; }
+int pv_storage(const PVArgs& pa, int vq, int rank, bool fused, int S) {
+  return vq == VQ_BLOCK && pv_block_ok(pa, rank, fused, S) ? VQ_RAW : vq;
+}
 
 int validate_decode(const starkv_decode_desc* d, int* gs, int* n_wg, int* k1pc, int* vq) {
   if (!d) return STARKV_ERR_NULL;
@@ -733,7 +735,7 @@ int validate_decode(const starkv_decode_desc* d, int* gs, int* n_wg, int* k1pc, 
   if (st) return st;
   PVArgs vtmp = {};
   if ((st = validate_v(d->v, vtmp, vq)) || (st = check_v_step(d->v, d->seq_len))) return st;
-  *vq = pv_storage(vtmp, *vq, d->v.rank);
+  *vq = pv_storage(vtmp, *vq, d->v.rank, true, d->seq_len);
   if (!d->q || !d->uv || !d->out || !d->rope_table) return STARKV_ERR_NULL;
   if (d->seq_len > d->rope_max_positions) return STARKV_ERR_SHAPE;
   if (d->uv_row_stride < d->v.rank) return STARKV_ERR_SHAPE;
@@ -1008,7 +1010,7 @@ size_t starkv_pv_latent_workspace_bytes(const starkv_pv_desc* d) {
   PVArgs tmp = {};
   int vq = 0;
   if (validate_v(d->v, tmp, &vq) || check_v_step(d->v, d->seq_len)) return 0;
-  vq = pv_storage(tmp, vq, d->v.rank);
+  vq = pv_storage(tmp, vq, d->v.rank, false, d->seq_len);
   const int BQ = d->batch * head_groups(d->n_heads);
   const PVGeom g = pv_geometry(BQ, d->seq_len, d->v.rank, false, vq, v_row_bytes(d->v));
   return a256((size_t)BQ * g.n_c2 * 32 * g.Rvp * 4) + a256((size_t)BQ * g.n_grp * 32 * g.Rvp * 4);
@@ -1022,7 +1024,7 @@ int starkv_pv_latent(const starkv_pv_desc* d, void* workspace, size_t workspace_
   int st, vq = 0;
   PVArgs a = {};
   if ((st = validate_v(d->v, a, &vq)) || (st = check_v_step(d->v, d->seq_len))) return st;
-  vq = pv_storage(a, vq, d->v.rank);
+  vq = pv_storage(a, vq, d->v.rank, false, d->seq_len);
   if (!d->p || !d->out) return STARKV_ERR_NULL;
   const size_t need = starkv_pv_latent_workspace_bytes(d);
   if (!workspace || workspace_bytes < need) return STARKV_ERR_WORKSPACE;
@@ -1083,7 +1085,7 @@ static int decode_impl(const starkv_decode_desc* d, void* workspace, size_t work
 
   PVArgs pa = {};
   if ((st = validate_v(d->v, pa, &vq))) return st;
-  vq = pv_storage(pa, vq, d->v.rank);
+  vq = pv_storage(pa, vq, d->v.rank, true, d->seq_len);
   pa.logits = (const float*)(ws + L.off_logits); pa.l_sb = ka.o_sb; pa.l_st = ka.o_st; pa.l_sh = ka.o_sh;
   pa.chunkmax = (const float*)(ws + L.off_cmax); pa.n_chunk1 = L.n_c1;
   pa.part = (float*)(ws + L.off_part); pa.psum = (float*)(ws + L.off_psum); pa.part16 = L.part16;

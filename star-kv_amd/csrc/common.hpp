@@ -430,7 +430,7 @@ int launch_k_logits_ws(const KArgs& a, int dtype, bool out_f32, int out_dtype, i
 int launch_k_logits_gqa(const KArgs& a, int dtype, bool out_f32, int out_dtype, int B, hipStream_t st);
 int launch_pv(const PVArgs& a, int dtype, int vq, bool fused, bool fast, int B, hipStream_t st);
 int pv_tiles_per_wave(int Rvp, bool fused, int vq);   // column tiles (of 32 ranks) per P.V wave
-bool pv_block_ok(const PVArgs& a, int Rv);           // the storage fields (validate_v) are set
+bool pv_block_ok(const PVArgs& a, int Rv, bool fused, int S);   // the storage fields (validate_v) are set
 int pv_wide_tiles(int Rvp, bool fused, int vq);       // > 0: the 8-wave all-columns kernel, tiles per wave
 // P.V workgroups resident per CU (the kernel's register budget): the wide
 // dense variants (8 and 13 tiles) take one, the others two

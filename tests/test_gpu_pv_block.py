@@ -27,6 +27,14 @@ def test_dequant_bit_exact(kind, R, split, pad, dtype):
     _dequant_one_hot(kind, R, split, dtype, pad)
 
 
+# rows of whole dwords past 1280 ranks: the context length at which the drop-in product changes kernels; unaligned ones
+@pytest.mark.parametrize("S", [2047, 2048])
+@pytest.mark.parametrize("kind,R,split,pad", [("int4_whole", 1640, 1640, 0), ("ref_int4", 1792, 512, 0), ("ref_int8", 1288, 256, 0),
+                                              ("ref_int4", 1288, 256, 1)])
+def test_many_ranks(kind, R, split, pad, S):
+    test_products(kind, R, split, pad, F16, 1, S, 8)
+
+
 @pytest.mark.parametrize("B,S,H", [(1, 1, 32), (2, 31, 8), (1, 33, 40), (3, 500, 32)])
 @pytest.mark.parametrize("kind,R,split,pad,dtype", [SHAPES[0] + (F16,), SHAPES[5] + (F16,), SHAPES[7] + (F16,), SHAPES[9] + (BF16,),
                                                     SHAPES[13] + (BF16,), SHAPES[14] + (F16,)])
