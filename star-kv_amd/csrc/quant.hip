@@ -519,28 +519,67 @@ static void launch_v_rows(const VAppendArgs& a, int dtype, hipStream_t st) {
   launch_block(k, dtype, st);
 }
 
-// The chunked kernels take over where their ~10 us of fixed time (two launches,
-// each a chain of loads, maxima and divisions) pays: from 16384 rows on
-// (positions x heads, or x 64-rank groups of V), 32768 unquantised.  Measured,
-// K and V written together, row-per-wave against chunked, us: 32 heads, int8 /
-// group-64: 512 positions 12.6 / 13.1, 2048 43.7 / 16.2, 16384 310 / 51;
-// dense: 512 8.8 / 10.4, 1024 12.5 / 11.1, 16384 142 / 39.  8 heads, int8 /
-// group-64: 2048 positions 13.5 / 14.2, 16384 93 / 24; dense: 2048 7.0 / 10.5,
-// 16384 41 / 20.  A workgroup holds 8 or more positions of one batch: runs of
-// fewer than 16 stay with the row-per-wave kernels.
-static bool many_rows(int B, int T, int per_pos, bool dense) {
-  return T >= 16 && (int64_t)B * T * per_pos >= (dense ? 32768 : 16384);
+// Where the chunked kernels take over, from modelled times in ns.  Each has 6
+// to 12 us of fixed time (a chain of loads, maxima and divisions, eight passes
+// over one workgroup's positions).  The row-per-wave kernels start in 2.8 us
+// and take 0.34 ns of the whole chip per row of K or 64-rank group of V (0.53
+// with a lower block, 0.21 unquantised); the one wave of a block or dense row
+// of V also takes 3.6 or 1.7 ns per rank, whatever the chip does beside it.
+// Measured, row-per-wave against chunked, us:
+//   K alone, 32 heads: int8 rank 48, 512 positions 8.4 / 8.3; rank 51, 768
+//   11.0 / 11.5; rank 8, 768 11.1 / 11.4; split, rank 48, 512 12.3 / 9.9;
+//   unquantised rank 51, 1024 9.1 / 8.3.
+//   V alone: group-64 R1640, 512 positions 6.6 / 6.0; split R1640, 4096 12.4 /
+//   12.9, 8192 22.7 / 18.8; split R512, 8192 10.0 / 11.4, 16384 15.6 / 14.0;
+//   split R2560, 512 12.8 / 10.0; dense R512, 16384 8.1 / 9.4, 32768 17.7 /
+//   14.1; dense R1640, 2048 6.5 / 6.5, 4096 11.1 / 8.0; dense R2560, 512 7.5 / 6.7.
+//   both, in one launch against two: 32 heads, int8 / group-64 R1640, rank 51,
+//   512 12.8 / 16.4, 1024 22.6 / 16.8; rank 8, R64, 1024 14.4 / 16.2, 2048 26.0
+//   / 16.3; 8 heads of rank 64, R512, 2048 13.6 / 14.7; unquantised rank 96,
+//   R2560, 1024 18.0 / 13.4.
+// A workgroup holds pp * 8 / KC positions of one batch, 2 at the fewest: runs
+// of fewer than 16 stay with the row-per-wave kernels.
+static int64_t k_waves_ns(const KAppendArgs& a) {
+  int64_t ps = 0;
+  for (int h = 0; h < a.H; ++h) ps += a.fmt == STARKV_FMT_DENSE ? 210 : a.rank[h] > a.split ? 530 : 335;
+  return ps * a.B * a.T / 1000;
 }
-static bool many_rows(const KAppendArgs& a) { return many_rows(a.B, a.T, a.H, a.fmt == STARKV_FMT_DENSE); }
-static bool many_rows(const VAppendArgs& a) { return many_rows(a.B, a.T, (int)ceil_div(a.R, 64), a.vq == VQ_DENSE); }
+static bool k_chunked(const KAppendArgs& a) {
+  if (a.T < 16) return false;
+  return a.fmt == STARKV_FMT_DENSE ? (int64_t)a.B * a.T * a.H >= 28672 : k_waves_ns(a) >= 8200;   // 24.5 K rows, 15.5 K with a lower block
+}
+static int64_t v_row_ns(const VAppendArgs& a) {
+  return 2800 + (a.vq == VQ_G64 ? 0 : a.vq == VQ_DENSE ? a.R * 17 / 10 : 600 + a.R * 36 / 10);
+}
+static int64_t v_waves_ns(const VAppendArgs& a) {
+  return 335 * (int64_t)a.B * a.T * (a.vq == VQ_G64 ? ceil_div(a.R, 64) : 1) / 1000;
+}
+static bool v_chunked(const VAppendArgs& a) {
+  const int64_t rows = (int64_t)a.B * a.T, groups = ceil_div(a.R, 64);
+  if (a.T < 16) return false;
+  const bool dense = a.vq == VQ_DENSE;
+  if (a.vq == VQ_G64 || groups >= (dense ? 40 : 28)) return rows * groups >= 16384;
+  if (dense && groups >= 25) return rows * groups >= 53248;
+  return rows >= 24576 || rows * groups >= (dense ? 196608 : 131072);
+}
+// K and V in launches of their own, either or both chunked
+static bool step_apart(const KAppendArgs& k, const VAppendArgs& v) {
+  const bool kc = k_chunked(k), vc = v_chunked(v), dense = k.fmt == STARKV_FMT_DENSE;
+  if (!kc && !vc) return false;
+  const int64_t kw = k_waves_ns(k), vw = v_waves_ns(v), vr = v_row_ns(v);
+  bool two = false;
+  for (int h = 0; h < k.H; ++h) two = two || (!dense && k.rank[h] > k.split);
+  const int64_t kt = !kc ? 2800 + kw : dense ? 6500 : two ? 12000 : 11000;
+  const int64_t vt = !vc ? vr + vw : v.vq == VQ_G64 ? 6000 : v.vq == VQ_DENSE ? 6500 : 10500;
+  return kt + vt <= vr + kw + vw;
+}
 
 int launch_step_append(const StepAppendArgs& a0, int dtype, hipStream_t st) {
   StepAppendArgs a = a0;
-  if (many_rows(a.k)) {
-    launch_block(a.k, dtype, st);
-    launch_v_rows(a.v, dtype, st);
-    if (a.has_rope) return launch_rope_apply(a.r, dtype, st);
-    return (int)hipGetLastError();
+  if (step_apart(a.k, a.v)) {
+    int e = launch_k_append(a.k, dtype, st);
+    if (!e) e = launch_v_append(a.v, dtype, st);
+    return !e && a.has_rope ? launch_rope_apply(a.r, dtype, st) : e;
   }
   a.v.gw = a.v.vq == VQ_G64 ? (int)ceil_div(a.v.R, 64) : 1;
   a.nbk = ceil_div((int64_t)a.k.B * a.k.H * a.k.T, 4);
@@ -556,7 +595,7 @@ int launch_step_append(const StepAppendArgs& a0, int dtype, hipStream_t st) {
 int launch_k_append(const KAppendArgs& a, int dtype, hipStream_t st) {
   const int64_t rows = (int64_t)a.B * a.H * a.T;
   if (rows == 0) return 0;
-  if (many_rows(a)) {
+  if (k_chunked(a)) {
     launch_block(a, dtype, st);
     return (int)hipGetLastError();
   }
@@ -569,7 +608,7 @@ int launch_k_append(const KAppendArgs& a, int dtype, hipStream_t st) {
 int launch_v_append(const VAppendArgs& a, int dtype, hipStream_t st) {
   const int64_t rows = (int64_t)a.B * a.T;
   if (rows == 0) return 0;
-  if (many_rows(a)) {
+  if (v_chunked(a)) {
     launch_v_rows(a, dtype, st);
     return (int)hipGetLastError();
   }

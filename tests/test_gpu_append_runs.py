@@ -18,6 +18,10 @@ SHAPES = [
     ("four_per_thread", [128] * 40, 4203, 3, 277),
     ("split_edges", [16, 17, 24, 128], 256, 8, 1030),
     ("split_edges_v", [3, 31], 263, 900, 21),
+    # V rows of one chunk per thread in the block kernel: past a rank's row count, past 28 groups
+    ("block_v", [16], 300, 30, 820),
+    ("block_v_split_edge", [8], 257, 25, 1000),
+    ("block_v_wide", [16, 9], 1793, 4, 4100),
 ]
 
 
