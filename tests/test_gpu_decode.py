@@ -232,7 +232,11 @@ LAST_POS_CASES = [
     # name, B, Hq, Hkv, S, ranks, Rv, layout: each K-logit kernel family
     ("mha_ws_dense", 2, 32, 32, 700, None, 256, "ragged"),
     ("gqa4_dense", 2, 32, 8, 700, [32, 128, 32, 80, 32, 64, 80, 64], 256, "ragged"),
-    ("unaligned_r_streaming", 2, 32, 32, 129, [20] * 32, 50, "reference"),
+    ("mha_ws_linear", 2, 32, 32, 129, [20] * 32, 50, "reference"),
+    # rows neither contiguous nor aligned: the register-streaming kernel
+    ("unaligned_r_streaming", 2, 8, 8, 129, [20, 33, 7, 64, 101, 16, 5, 90], 50, "posmajor"),
+    ("unaligned_r_streaming_gqa", 2, 12, 4, 300, [33, 48, 7, 101], 50, "posmajor"),
+    ("gqa_linear", 2, 16, 4, 333, [102, 49, 127, 9], 256, "ragged"),
 ]
 
 

@@ -96,3 +96,50 @@ def test_dense_v_rows(Rv, B, S, pad, dtype):
     check_output(pv_latent(p, xv), ref, "P.V ")
     out = decode_attention(case.q, case.kspec, xv, case.uv, out_dtype=torch.float32)
     check_output(out, oracle_decode(case)[0], "decode ")
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("ranks,S", [([102, 49, 127, 9], 333), ([8, 33, 64, 119], 32), ([31, 95], 2049)])
+def test_gqa_linear_rows_masked(ranks, S, dtype):
+    """Grouped queries over contiguous odd ranks under an additive mask and
+    under a device-held last position, contexts ending inside a tile: both
+    against the oracle, and the two forms of the same mask against each other."""
+    from starkv import decode_attention, k_logits
+    B, Hkv = 2, len(ranks)
+    print(f"[gqa linear masked] {ranks} S={S} {dtype}", flush=True)
+    case = make_case(B, 4 * Hkv, Hkv, S, ranks, 64, dtype=dtype, seed=16)
+    last, scale = S - 1 - S // 5, 128 ** -0.5
+    mask = torch.zeros(B, 1, S, device="cuda")
+    mask[..., last + 1:] = -1e30
+    mask[0, 0, :last + 1:7] = -3.0
+    out = decode_attention(case.q, case.kspec, case.xv, case.uv, mask=mask, out_dtype=torch.float32)
+    check_output(out, oracle_decode(case, mask=mask.double().cpu())[0], "additive mask ")
+    got = k_logits(case.q, case.kspec, S, scale=scale, mask=mask)
+    plain = k_logits(case.q, case.kspec, S, scale=scale)
+    # scale * sum + mask rounds once in the kernel (a fused multiply-add), scale * sum first here: at most half a unit in
+    # the last place of the product, and one of the result
+    assert bool(((got - (plain + mask)).abs() <= 2.0 ** -23 * (plain.abs() + (plain + mask).abs())).all())
+    mask[0, 0, :last + 1] = 0.0
+    lp = torch.tensor([last], dtype=torch.int32, device="cuda")
+    a = decode_attention(case.q, case.kspec, case.xv, case.uv, last_pos=lp, out_dtype=torch.float32)
+    m = decode_attention(case.q, case.kspec, case.xv, case.uv, mask=mask, out_dtype=torch.float32)
+    check_output(a, oracle_decode(case, mask=mask.double().cpu())[0], "last position ")
+    # (past the last position -1e30 against a logit plus -1e30: the same fp32 number)
+    assert torch.equal(a, m)
+
+
+@pytest.mark.parametrize("latent_scale,q_scale", [(30000.0, 1.0), (1.0, 1e5), (3000.0, 3e4)], ids=["keys", "queries", "both"])
+def test_gqa_linear_bf16_beyond_fp16_range(latent_scale, q_scale):
+    """bf16 keys or queries past fp16's range over contiguous odd ranks: the
+    rerun with scaled keys (test_gpu_decode.py has it for aligned rows)."""
+    from starkv import k_logits
+    ranks = [101, 102, 33, 127, 49, 64, 97, 15]
+    case = make_case(1, 32, 8, 300, ranks, 64, dtype=BF16, seed=17, latent_scale=latent_scale)
+    case.q.mul_(q_scale)
+    print(f"[gqa linear bf16 range] {latent_scale} {q_scale}", flush=True)
+    out = k_logits(case.q, case.kspec, 300)
+    ref = oracle_logits(case)
+    assert torch.isfinite(out).all()
+    rms = float(ref.pow(2).mean().sqrt())
+    d = (out.double().cpu() - ref).abs() / rms
+    assert float(d.max()) <= 2e-2 and float(d.mean() / (ref.abs().mean() / rms)) <= 1e-3
