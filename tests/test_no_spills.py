@@ -4,12 +4,16 @@ A VGPR spill inside a K-step or tile loop is a scratch round trip, and the
 reload's memory wait also waits for the loop's own stores and loads: one
 spilled 64-bit address in the int8 warp-specialised K-logit kernel cost 11 %
 of its time at B16 S32768.  This test compiles the hot-path sources to
-gfx950 assembly with the library's flags and fails if any of their kernels
-that the decode path runs on aligned inputs reports a VGPR spill:
+gfx950 assembly with the library's flags and fails if any of these kernels
+reports a VGPR spill:
 * every instantiation of the warp-specialised and grouped-query K-logit
-  kernels, the raw-nibble P.V kernel and the split-S reduction / up-projection;
-* the fused, aligned-row column-block P.V kernel for dense and group-64 V.
-(The unaligned-row and per-token block-format P.V variants are not covered.)
+  kernels, the raw-nibble and per-token block-format P.V kernels and the
+  split-S reduction / up-projection;
+* the column-block P.V kernel for dense V of any alignment, and fused for
+  aligned group-64 V;
+* the cache writer's chunked kernels and the causal prefill attention.
+(Not covered: the dequantise-first P.V kernels for block formats and for
+unaligned group-64 rows, some of whose wide variants do spill.)
 """
 import concurrent.futures
 import os
@@ -29,10 +33,14 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-tar
 CHECKS = [
     ("k_logits_ws.hip", r"k_logits_ws_kernel"),
     ("k_logits_gqa.hip", r"k_logits_gqa_kernel"),
-    ("pv_latent.hip", r"pv_nib_kernel"),
+    ("pv_latent.hip", r"pv_nib_kernel|pv_block_kernel"),
     # pv_kernel<VT, NTW, FUSED = true, FAST = true, VQ = dense (0) or group-64 (2)>
     ("pv_latent.hip", r"pv_kernelI(DF16_|DF16b)Li\d+ELb1ELb1ELi[02]E"),
+    # pv_kernel<VT, NTW, FUSED, FAST = false, VQ = dense>
+    ("pv_latent.hip", r"pv_kernelI(DF16_|DF16b)Li\d+ELb[01]ELb0ELi0E"),
     ("up_proj.hip", r"up_proj_kernel|up_finish_kernel"),
+    ("quant.hip", r"append_(block|g64)_kernel"),
+    ("prefill.hip", r"fa_causal_kernel"),
 ]
 
 
