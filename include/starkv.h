@@ -114,7 +114,11 @@ int starkv_rope_apply(const starkv_rope_apply_desc* d, void* stream);
  * streaming K-logit kernels cannot read (neither contiguous nor 16-byte
  * aligned with a rank that is a multiple of 8) are copied by starkv_k_logits
  * into its workspace first; quantised rows of any byte alignment are read as aligned
- * words joined in registers.
+ * words joined in registers.  Memory is read in whole aligned pieces that hold
+ * at least one byte of a row: dense contiguous rows and INT8_SYM rows in pieces
+ * of 16 bytes (so up to 14 bytes before a head's first row and after its last
+ * may be read), other quantised rows in pieces of 4.  What lies there never
+ * reaches a result.
  * Quantised K (offsets and strides of data/data2 in bytes; every value
  * dequantised to fp16 before use, as the reference's
  * dequantise-then-multiply path does, LlamaLoRaAttention_headwise_quant.py:

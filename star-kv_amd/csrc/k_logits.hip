@@ -209,9 +209,12 @@ __global__ __launch_bounds__(NW * 64, 1) void k_logits_kernel(const KArgs a) {
   // Tiles are processed in groups of G (a multiple of the 3-tile latent
   // register ring) per staging barrier.  Every
   // index is clamped to the chunk's last tile, so a group past the end
-  // re-reads that tile (cached) and only its stores are predicated off: the
-  // group body has no data-dependent branches and the compiler keeps the
-  // latent loads two tiles ahead of their use.
+  // re-reads that tile (cached) and only its stores are predicated off.  For
+  // aligned dense rows the group body then has no data-dependent branches and
+  // the compiler keeps the latent loads two tiles ahead of their use; the
+  // loads of quantised latents sit in per-lane branches (int8 or int4 block,
+  // dword-aligned or not) and those of unaligned dense rows in per-element
+  // ones, and there it waits for every load in flight at each item.
   const int last = tile1 - 1;
   const int n_groups = (tile1 - tile0 + G - 1) / G;
 
