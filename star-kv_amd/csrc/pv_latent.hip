@@ -185,7 +185,12 @@ __device__ inline void store_tile_f16(_Float16* out, int64_t pitch, int col0, co
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int v = 4 * g + 2 * i, q = 8 * g + 4 * hh + 2 * i;
-      const h2v h = {(_Float16)(acc[v] * inv[q]), (_Float16)(acc[v + 1] * inv[q + 1])};
+      // products rounded once, to fp16: left to itself the compiler converts
+      // the pair together and rounds each to fp32 first (the empty asm keeps
+      // the two apart)
+      uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)(acc[v] * inv[q]));
+      asm("" : "+v"(lo));
+      const h2v h = {__builtin_bit_cast(_Float16, (uint16_t)lo), (_Float16)(acc[v + 1] * inv[q + 1])};
       const uint32_t own = as_u32(h), other = quad_xor<1>(own);
       p[i] = __builtin_amdgcn_perm(own, other, sel);
     }

@@ -63,14 +63,34 @@ def _compile(src, tmp_path):
     return src, out.read_text()
 
 
-@pytest.mark.skipif(not shutil.which(HIPCC) and not os.path.exists(HIPCC), reason="hipcc not installed")
-def test_hot_path_kernels_do_not_spill(tmp_path):
+@pytest.fixture(scope="module")
+def asm(tmp_path_factory):
+    if not shutil.which(HIPCC) and not os.path.exists(HIPCC):
+        pytest.skip("hipcc not installed")
+    tmp_path = tmp_path_factory.mktemp("asm")
     srcs = sorted({s for s, _ in CHECKS})
     with concurrent.futures.ThreadPoolExecutor(len(srcs)) as ex:
-        asm = dict(ex.map(lambda s: _compile(s, tmp_path), srcs))
+        return dict(ex.map(lambda s: _compile(s, tmp_path), srcs))
+
+
+def test_hot_path_kernels_do_not_spill(asm):
     bad = []
     for src, pat in CHECKS:
         found = {k: v for k, v in _spills(asm[src]).items() if re.search(pat, k)}
         assert found, f"no kernel of {src} matches {pat}"
         bad += [(k, v) for k, v in found.items() if v]
     assert not bad, f"VGPR spills in hot-path kernels: {bad}"
+
+
+def test_fp16_partials_are_rounded_once(asm):
+    """The fused P.V kernels store fp16(sum * reciprocal), rounded once by a
+    mixed-precision multiply-add.  Packing two of them into one word invites the
+    compiler to form both products in fp32 and convert the pair, rounding twice."""
+    found = 0
+    for m in re.finditer(r"^(_ZN6starkv\d+(?:pv_nib|pv_block)_kernel\S+):.*?$(.*?)^\.Lfunc_end", asm["pv_latent.hip"], re.M | re.S):
+        name, body = m.groups()
+        if "pv_block" in name and not re.search(r"Li\d+ELi\d+ELb1E", name):
+            continue                                   # the drop-in form keeps fp32 partials
+        found += 1
+        assert "v_fma_mixlo_f16" in body and "v_cvt_pk_f16_f32" not in body, name
+    assert found == 14, found
