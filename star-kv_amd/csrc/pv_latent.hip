@@ -147,8 +147,7 @@ __device__ inline uint4 f16x8_to_bf16x8(uint4 h) {
 
 // the maximum of one head's K1 chunk maxima cm[0, n) over c = j, j+8, ...
 // (j < 8): eight independent loads in flight per step, clamped to the last
-// chunk in the last one (a load-then-max loop waits out one memory latency per
-// chunk, ~2 us each: the maxima were just written by other XCDs)
+// chunk in the last one
 __device__ inline float chunk_max_part(const float* cm, int n, int j) {
   float m = -INFINITY;
   for (int c = j; c < n; c += 64) {
@@ -162,41 +161,18 @@ __device__ inline float chunk_max_part(const float* cm, int n, int j) {
 }
 
 // One 32 x 32 accumulator tile (lane (n, hh) holds column n of rows
-// 8 g + 4 hh + i, g, i < 4), each row times inv[row] (in LDS) and rounded to
-// fp16, to a row-major array of row pitch `pitch` at column col0: the four
-// lanes of a quad exchange four rows of their four columns, so that lane n
-// stores columns n & ~3 .. + 3 of row 8 g + 4 hh + n % 4 with one instruction.
-// A store takes the address unit a cycle per four lanes whatever its width:
-// 112 2-byte stores per wave spent 6 us of a 29 us launch (B4 S4099 Rv 1640,
-// 128-position chunks; 23 us with these).  fp32 partials gain nothing from it
-// (their dwords already fill the data path; measured 1 us slower).
-template <int SEL> __device__ inline uint32_t quad_xor(uint32_t v) {
-  static_assert(SEL == 1 || SEL == 2, "a lane of the quad");
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, SEL == 1 ? 0xB1 : 0x4E, 0xF, 0xF, true);
-}
+// 8 g + 4 hh + i, g, i < 4), each row times inv[row] (in LDS, formed once per
+// workgroup) and rounded once to fp16, to a row-major array of row pitch
+// `pitch` at column col0.  One 2-byte store per value, 64 bytes a row half:
+// rows exchanged among the lanes of a quad for 8-byte stores were slower (B8
+// S8449 Rv 1640: decode call 102.6 us, 106.0 with them; split caches, B4
+// S4099: 71.1 and 75.4; Rv 2048, S300: 42.2 and 47.1).
 __device__ inline void store_tile_f16(_Float16* out, int64_t pitch, int col0, const floatx16& acc, const float* inv, int lane) {
   const int n = lane & 31, hh = lane >> 5;
-  const bool b1 = n & 2;
-  // even lanes keep the low halves (row i) of themselves and of lane n ^ 1, odd lanes the high ones (row i + 1)
-  const uint32_t sel = (n & 1) ? 0x07060302u : 0x01000504u;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    uint32_t p[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int v = 4 * g + 2 * i, q = 8 * g + 4 * hh + 2 * i;
-      // products rounded once, to fp16: left to itself the compiler converts
-      // the pair together and rounds each to fp32 first (the empty asm keeps
-      // the two apart)
-      uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)(acc[v] * inv[q]));
-      asm("" : "+v"(lo));
-      const h2v h = {__builtin_bit_cast(_Float16, (uint16_t)lo), (_Float16)(acc[v + 1] * inv[q + 1])};
-      const uint32_t own = as_u32(h), other = quad_xor<1>(own);
-      p[i] = __builtin_amdgcn_perm(own, other, sel);
-    }
-    const uint32_t got = quad_xor<2>(b1 ? p[0] : p[1]);
-    const uint2 w = b1 ? make_uint2(got, p[1]) : make_uint2(p[0], got);
-    *(uint2*)(out + (int64_t)(8 * g + 4 * hh + (n & 3)) * pitch + col0 + (n & ~3)) = w;
+  for (int v = 0; v < 16; ++v) {
+    const int q = 8 * (v >> 2) + 4 * hh + (v & 3);
+    out[q * pitch + col0 + n] = (_Float16)(acc[v] * inv[q]);
   }
 }
 
@@ -1176,7 +1152,7 @@ __global__ __launch_bounds__(NWV * 64, (PVNGeom<NWV, NGW, D16>::WGS)) void pv_ni
     copy(V2, 2);
     load(R[0], 0);
     load(R[1], 1);
-    // the heads' maxima, their latency under the first copies'
+    // the heads' maxima (before or after the first copies: the same time)
     if (tid < 256) {
       const int q = tid >> 3, j = tid & 7;
       float m = -INFINITY;

@@ -84,8 +84,8 @@ def test_hot_path_kernels_do_not_spill(asm):
 
 def test_fp16_partials_are_rounded_once(asm):
     """The fused P.V kernels store fp16(sum * reciprocal), rounded once by a
-    mixed-precision multiply-add.  Packing two of them into one word invites the
-    compiler to form both products in fp32 and convert the pair, rounding twice."""
+    mixed-precision multiply-add.  Packed in pairs, the compiler has formed both
+    products in fp32 and converted the pair, rounding twice."""
     found = 0
     for m in re.finditer(r"^(_ZN6starkv\d+(?:pv_nib|pv_block)_kernel\S+):.*?$(.*?)^\.Lfunc_end", asm["pv_latent.hip"], re.M | re.S):
         name, body = m.groups()
