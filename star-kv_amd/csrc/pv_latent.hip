@@ -1494,13 +1494,11 @@ __global__ __launch_bounds__(512, 1) void pv_block_kernel(const PVArgs a) {
 // kernel's registers hold (an int8 latent past 1024 ranks has too many),
 // 24-bit row pitches.  The others keep pv_wide_kernel and pv_kernel.
 //
-// So do rows of whole dwords past 1280 ranks where those are as fast or
-// faster: int4 upper blocks in the decode call (calls of 1792 int4 ranks, B16
-// S2048: 82.6 us raw, 80.0 before; B1 S4099: 59.9 and 58.9; int8 uppers gain 2
-// to 10 %), and every kind in the drop-in product of short contexts (R1792,
-// S300: 12.9 and 12.0; B3 S5003: 33.8 raw, 37.5 before).  Decided by ranks and
-// pitches alone, so that the workspace a shape asks for does not depend on a
-// buffer's address.
+// So do rows of whole dwords past 1280 ranks in the drop-in product of short
+// contexts (1792 int4 ranks: S300 12.9 us raw, 12.0 before; B3 S5003 33.7 and
+// 37.8; the decode call gains at every length: S300 41.2 and 44.8, B16 S2048
+// 76.6 and 78.1).  Decided by ranks and pitches alone, so that the workspace a
+// shape asks for does not depend on a buffer's address.
 bool pv_block_ok(const PVArgs& a, int Rv, bool fused, int S) {
   const bool two = a.split < Rv;
   if (Rv > PVB_MAX_RV || (two && a.split % 32)) return false;
@@ -1508,7 +1506,7 @@ bool pv_block_ok(const PVArgs& a, int Rv, bool fused, int S) {
   const int up = a.a_int8 ? 8 : 4;
   const bool dwords = a.split % 8 == 0 && a.x_ss % up == 0 && a.x_sb % up == 0 &&
                       (!two || ((Rv - a.split) % 8 == 0 && a.x2_ss % 4 == 0 && a.x2_sb % 4 == 0));
-  if (Rv > 1280 && dwords && (fused ? !a.a_int8 : S < 2048)) return false;
+  if (Rv > 1280 && dwords && !fused && S < 2048) return false;
   const int pieces = pvb_pieces(a.xnb) + (two ? pvb_pieces(a.x2nb) : 0);
   return pieces <= pvb_max_pieces(pvb_tiles((int)round_up(Rv, 32))) && a.x_ss < (1 << 24) && (!two || a.x2_ss < (1 << 24));
 }
