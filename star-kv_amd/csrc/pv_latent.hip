@@ -1492,13 +1492,17 @@ __global__ __launch_bounds__(512, 1) void pv_block_kernel(const PVArgs a) {
 // Whether the block formats' raw kernel takes this latent: whole tiles in the
 // upper block, rows of at least one 16-byte piece and no more than the
 // kernel's registers hold (an int8 latent past 1024 ranks has too many),
-// 24-bit row pitches.  The others keep pv_wide_kernel and pv_kernel.
+// 24-bit row pitches.  The others keep pv_wide_kernel and pv_kernel.  Few
+// ranks, of which some waves own no tile, gain too: 168 calls of 32 to 224
+// ranks run at 1.17 times the others' speed in the geometric mean, at 0.97 at
+// the slowest (32 ranks, S65536: 15.7 us raw, 15.2 before).
 //
-// So do rows of whole dwords past 1280 ranks in the drop-in product of short
-// contexts (1792 int4 ranks: S300 12.9 us raw, 12.0 before; B3 S5003 33.7 and
-// 37.8; the decode call gains at every length: S300 41.2 and 44.8, B16 S2048
-// 76.6 and 78.1).  Decided by ranks and pitches alone, so that the workspace a
-// shape asks for does not depend on a buffer's address.
+// Rows of whole dwords past 1280 ranks keep the others in the drop-in product
+// of short contexts (1792 int4 ranks: S300 12.9 us raw, 12.0 before; B3 S5003
+// 33.7 and 37.8; the decode call gains at every length: S300 41.2 and 44.8,
+// B16 S2048 76.6 and 78.1).  Decided by ranks, pitches and the context's length
+// alone, so that the workspace a shape asks for does not depend on a buffer's
+// address.
 bool pv_block_ok(const PVArgs& a, int Rv, bool fused, int S) {
   const bool two = a.split < Rv;
   if (Rv > PVB_MAX_RV || (two && a.split % 32)) return false;
